@@ -50,8 +50,7 @@ HZK_DEV uint32_t find_key(const uint32_t* __restrict__ offs, uint32_t nk, uint32
 // to bucket[k]; the partial of a bucket that began in an earlier chunk goes
 // to carry[2c] (head), that of a bucket continuing into the next chunk to
 // carry[2c+1] (tail). Persistent grid over the whole batch's chunk space.
-// G1: the additions in 29-bit-limb arithmetic (field29.hpp: one
-// v_mad_u64_u32 per partial product, lazy reduction) over the bases converted
+// G1: the additions in 29-bit-limb arithmetic (field29.hpp) over the bases converted
 // to its Montgomery form by k_msm_convert_g1. Bucket sums and chunk partials
 // are stored as raw accumulator states (g1acc29::store_raw), the form the
 // fix-up and the bucket reduction work in. At least two waves per SIMD (the
@@ -98,9 +97,7 @@ static __global__ void __launch_bounds__(256, 2) k_msm_accumulate_g1(MsmBatchDev
                 p0 = bp[0], p1 = bp[1], p2 = bp[2], p3 = bp[3];
             }
             if (!inf) {
-                const fq29 x = fq29::unpack(x0, x1), ya = fq29::unpack(y0, y1);
-                const fq29 y = neg ? fq29::neg(ya, fq29::P1) : ya;
-                acc.add_affine(x, y);
+                acc.add_affine(fq29::unpack(x0, x1), fq29::negate_if(fq29::unpack(y0, y1), neg));
             }
             if (e + 1 == next || e + 1 == e1) {
                 if (before) acc.store_raw(carry + RW * (2 * gid));
@@ -155,9 +152,8 @@ static __global__ void __launch_bounds__(256, 2) k_msm_accumulate_g2(MsmBatchDev
             }
             if (p3.w != 0xffffffffu) {   // the converter's mark for the point at infinity
                 const fq2_29 x{fq29::unpack(p0, p1), fq29::unpack(p2, p3)};
-                fq2_29 y{fq29::unpack(p4, p5), fq29::unpack(p6, p7)};
-                if (neg) y = {fq29::neg(y.c0, fq29::P1), fq29::neg(y.c1, fq29::P1)};
-                acc.add_affine(x, y);
+                const fq2_29 y{fq29::unpack(p4, p5), fq29::unpack(p6, p7)};
+                acc.add_affine(x, fq2_29::negate_if(y, neg));
             }
             if (e + 1 == next || e + 1 == e1) {
                 if (before) acc.store_raw(carry + RW * (2 * gid));
@@ -197,8 +193,9 @@ HZK_DEV void convert_point_g1(const uint4* __restrict__ sp, uint4* __restrict__ 
     const uint32_t xw[8] = {a.x, a.y, a.z, a.w, b2.x, b2.y, b2.z, b2.w};
     const uint32_t yw[8] = {c.x, c.y, c.z, c.w, e.x, e.y, e.z, e.w};
     uint32_t xo[8], yo[8];
+    const fq29 xi = fq29::unpack(xw), yi = fq29::unpack(yw), to = fq29::konst(fq29::TO);
     fq29 x, y;
-    fq29::mul2(x, fq29::unpack(xw), fq29::konst(fq29::TO), y, fq29::unpack(yw), fq29::konst(fq29::TO));
+    scan29(Mul29<Fq29Mod>(x, xi, to), Mul29<Fq29Mod>(y, yi, to));
     x.canonical().pack(xo);
     y.canonical().pack(yo);
     dp[0] = make_uint4(xo[0], xo[1], xo[2], xo[3]);
@@ -227,8 +224,9 @@ HZK_DEV void convert_point_g2(const uint4* __restrict__ sp, uint4* __restrict__ 
         const uint32_t a[8] = {v[2 * c].x, v[2 * c].y, v[2 * c].z, v[2 * c].w, v[2 * c + 1].x, v[2 * c + 1].y, v[2 * c + 1].z, v[2 * c + 1].w};
         const uint32_t b[8] = {v[2 * c + 2].x, v[2 * c + 2].y, v[2 * c + 2].z, v[2 * c + 2].w,
                                v[2 * c + 3].x, v[2 * c + 3].y, v[2 * c + 3].z, v[2 * c + 3].w};
+        const fq29 xi = fq29::unpack(a), yi = fq29::unpack(b), to = fq29::konst(fq29::TO);
         fq29 x, y;
-        fq29::mul2(x, fq29::unpack(a), fq29::konst(fq29::TO), y, fq29::unpack(b), fq29::konst(fq29::TO));
+        scan29(Mul29<Fq29Mod>(x, xi, to), Mul29<Fq29Mod>(y, yi, to));
         uint32_t xo[8], yo[8];
         x.canonical().pack(xo);
         y.canonical().pack(yo);
@@ -580,22 +578,16 @@ template <class F>
 HZK_DEV acc29_t<F> acc_from_xyzz(const xyzz_t<F>& p);
 template <>
 HZK_DEV g1acc29 acc_from_xyzz<fq_t>(const xyzz_t<fq_t>& p) {
-    g1acc29 a;
-    a.inf = p.ZZ.is_zero();
-    fq29::mul2(a.X, fq29::unpack(p.X.l), fq29::konst(fq29::TO), a.Y, fq29::unpack(p.Y.l), fq29::konst(fq29::TO));
-    fq29::mul2(a.ZZ, fq29::unpack(p.ZZ.l), fq29::konst(fq29::TO), a.ZZZ, fq29::unpack(p.ZZZ.l), fq29::konst(fq29::TO));
-    return a;
+    auto to = [](const fq_t& v) { return fq29::mul(fq29::unpack(v.l), fq29::konst(fq29::TO)); };
+    return {to(p.X), to(p.Y), to(p.ZZ), to(p.ZZZ), p.ZZ.is_zero()};
 }
 template <>
 HZK_DEV g2acc29 acc_from_xyzz<fq2_t>(const xyzz_t<fq2_t>& p) {
-    g2acc29 a;
-    a.inf = p.ZZ.is_zero();
-    const fq29 T = fq29::konst(fq29::TO);
-    fq29::mul2(a.X.c0, fq29::unpack(p.X.c0.l), T, a.X.c1, fq29::unpack(p.X.c1.l), T);
-    fq29::mul2(a.Y.c0, fq29::unpack(p.Y.c0.l), T, a.Y.c1, fq29::unpack(p.Y.c1.l), T);
-    fq29::mul2(a.ZZ.c0, fq29::unpack(p.ZZ.c0.l), T, a.ZZ.c1, fq29::unpack(p.ZZ.c1.l), T);
-    fq29::mul2(a.ZZZ.c0, fq29::unpack(p.ZZZ.c0.l), T, a.ZZZ.c1, fq29::unpack(p.ZZZ.c1.l), T);
-    return a;
+    auto to = [](const fq2_t& v) -> fq2_29 {
+        const fq29 k = fq29::konst(fq29::TO);
+        return {fq29::mul(fq29::unpack(v.c0.l), k), fq29::mul(fq29::unpack(v.c1.l), k)};
+    };
+    return {to(p.X), to(p.Y), to(p.ZZ), to(p.ZZZ), p.ZZ.is_zero()};
 }
 
 template <class F>
