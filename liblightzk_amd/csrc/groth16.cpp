@@ -467,9 +467,9 @@ int g16_msm_batch(hzk_ctx* ctx, G16Req* reqs, size_t n, int graph) {
 }
 
 // Upper bound of one MSM's scratch (digits and sorted entries, histograms,
-// key scans, bucket sums, chunk partials, bucket-reduction and window sums)
-// for n points with xyzz points of pt_bytes (bucket sums, chunk partials and
-// run sums are raw 29-bit accumulator states, 9/8 of that), from the
+// key scans, bucket sums, chunk partials, window sums)
+// for n points with xyzz points of pt_bytes (bucket sums and chunk partials
+// are raw 29-bit accumulator states, 9/8 of that), from the
 // built-in plans (the larger of the single-MSM and wide-batch regimes).
 static size_t msm_scratch_bound(size_t n, size_t pt_bytes) {
     const size_t raw = pt_bytes / 8 * 9;
@@ -478,11 +478,10 @@ static size_t msm_scratch_bound(size_t n, size_t pt_bytes) {
         const MsmPlan p = msm_plan_builtin(pt_bytes > 128, n, regime, 160 * 1024);
         size_t W = p.W, nk = W * p.NB, entries = n * W;
         size_t chunks = (entries + p.K - 1) / p.K;
-        size_t bred = W * ((p.NB + p.g - 1) / p.g);
         const size_t coarse = p.NB >= 2048 && n >= MSM_TP_BATCH_MIN_N ? entries * 8 : 0;   // two-pass staging
         size_t b = entries * 8 + coarse + (size_t)p.T * nk * 4 + 2 * (nk + 1) * 4 +
                    2 * ((nk + 1 + MSM_SCAN_TILE) / MSM_SCAN_TILE) * 8 + (nk + 1) * raw + chunks * (4 + 2 * raw) +
-                   2 * bred * raw + 2 * 64 * W * pt_bytes + 4096;   // run (A, R) and part (P, RS) pairs
+                   W * raw + 2 * 64 * W * pt_bytes + 4096;   // window values, part (P, RS) pairs
         worst = std::max(worst, b);
     }
     return worst;

@@ -51,7 +51,7 @@ enum MsmSpace {
     SP_KEY,         // nk + 1 entries per instance (counts, offsets, bucket sums)
     SP_SCANTILE,    // scan tiles over the key space
     SP_CHUNK,       // accumulation chunks of K sorted entries (upper bound)
-    SP_BRED,        // bucket-reduction lanes (window x run)
+    SP_BRED,        // window values (device-side combine)
     SP_WIN,         // window-sum partials (S per window)
     SP_ENTRY,       // n * W digit / sorted-entry slots
     SP_HIST,        // T * nk per-tile histogram counters
@@ -65,7 +65,6 @@ struct MsmInst {
     const void* bases;     // affine points
     uint32_t n, c, W, NB, nk, K, g, G, T, tile;
     uint32_t S;            // window-sum workgroups per window
-    uint32_t fused;        // 1: each window-sum thread reduces one run of g buckets itself (no run-sum pass)
     // Level tables: nd scalars with Wd digit windows over a table of Lg levels
     // (point t*nd + i = 2^(c t) P_i, t < Lg); each bucket set ("window" of the
     // pipeline) serves Lg consecutive digit windows, so W = ceil(Wd / Lg) and

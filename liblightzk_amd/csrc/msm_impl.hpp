@@ -11,16 +11,13 @@
 #include "field29.hpp"
 #include "host_ec.hpp"
 #include "host_pool.hpp"
+#include "lanes29.hpp"
 #include "msm.hpp"
 
 namespace hzk {
 
-// fan-in of the tree over a hot bucket's chunk partials: each level is a
-// chain of K2 - 1 dependent additions on few lanes, so latency, not work,
-// sets its cost (4: three additions per level)
-static constexpr int K2 = 4;
-static constexpr uint32_t HOT = 16;  // a bucket spanning more chunks than this uses the tree
-static constexpr uint32_t HOT_LIST = 256;   // hot instances a hot-tree block lists in LDS
+static constexpr uint32_t HOT = 16;         // a bucket spanning more chunks than this is summed by k_msm_hot_sum first
+static constexpr uint32_t HOT_LIST = 256;   // hot instances a hot-sum block lists in LDS
 
 HZK_DEV uint32_t find_inst_g(const uint64_t* __restrict__ beg, uint32_t ninst, uint64_t gid) {
     uint32_t lo = 0, hi = ninst;
@@ -282,47 +279,49 @@ template <> struct Acc29<fq2_t> { using A = g2acc29; };
 template <class F> using acc29_t = typename Acc29<F>::A;
 template <class F> constexpr int raw_vec() { return acc29_t<F>::RAW_WORDS / 4; }
 
-// hot buckets (more than HOT chunks): one level of an in-place K2-ary tree
-// over the head partials carry[2c] of chunks f+1..l (f, l: first and last
-// chunk of the bucket); afterwards carry[2(f+1)] holds their sum
+// Hot buckets (more than HOT chunks): the head partials carry[2c] of chunks
+// f+1..l (f, l: first and last chunk of the bucket) are summed in place,
+// HOT_SEG slots' worth of them per workgroup and level, into the segment's
+// first; one or two levels leave the whole sum in carry[2(f+1)].
+template <class F> constexpr uint32_t hot_seg() { return 16 * LdsLanes<F, 256>::SLOTS; }
+
+// the segment starting at chunk c of instance ii at this level, or 0: number
+// of elements (stride chunks apart)
 template <class F>
-HZK_DEV void hot_tree_chunk(const MsmBatchDev& b, const uint32_t* __restrict__ offs, const uint32_t* __restrict__ chunk2key,
-                            uint32_t stride, uint4* __restrict__ carry, uint32_t ii, uint32_t c) {
-    using A = acc29_t<F>;
-    constexpr int RW = raw_vec<F>();
+HZK_DEV uint32_t hot_segment(const MsmBatchDev& b, const uint32_t* __restrict__ offs, const uint32_t* __restrict__ chunk2key,
+                             uint64_t stride, uint32_t ii, uint32_t c) {
     const MsmInst& d = b.inst[ii];
-    if ((uint64_t)c * d.K >= b.stats[4 * ii]) return;
-    const uint64_t* cbeg = space_g(b, SP_CHUNK);
+    if ((uint64_t)c * d.K >= b.stats[4 * ii]) return 0;
     const uint32_t* of = offs + space_g(b, SP_KEY)[ii];
-    const uint32_t k = chunk2key[cbeg[ii] + c], start = of[k];
-    if (start >= c * d.K) return;   // chunk c holds no head partial
+    const uint32_t k = chunk2key[space_g(b, SP_CHUNK)[ii] + c], start = of[k];
+    if (start >= c * d.K) return 0;   // chunk c holds no head partial
     const uint32_t f = start / d.K, l = (of[k + 1] - 1) / d.K;
-    if (l - f <= HOT) return;
-    const uint32_t rel = c - (f + 1), span = l - f;
-    if (rel % (stride * K2) != 0) return;
-    uint4* base = carry + (size_t)RW * 2 * cbeg[ii];
-    A acc = A::load_raw(base + (size_t)RW * 2 * c);
-    for (int i = 1; i < K2; ++i) {
-        uint32_t r = rel + i * stride;
-        if (r >= span) break;
-        acc.add(A::load_raw(base + (size_t)RW * 2 * (c + i * stride)));
-    }
-    acc.store_raw(base + (size_t)RW * 2 * c);
+    if (l - f <= HOT) return 0;
+    const uint64_t rel = c - (f + 1), span = l - f;
+    if (rel % (stride * hot_seg<F>()) != 0) return 0;
+    const uint64_t left = (span - rel + stride - 1) / stride;
+    return (uint32_t)(left < hot_seg<F>() ? left : hot_seg<F>());
 }
 
 template <class F>
-__global__ void __launch_bounds__(256) k_msm_hot_tree(MsmBatchDev b, const uint32_t* __restrict__ offs,
-                                                      const uint32_t* __restrict__ chunk2key, uint32_t stride,
-                                                      uint4* __restrict__ carry) {
-    // Most instances have no hot bucket. Each block lists the instances that
-    // do (largest bucket > HOT chunks), in instance order, with the prefix
-    // sums of their chunk counts, all in LDS; the grid then strides over the
-    // concatenated chunks of the hot instances only, one (instance, chunk)
-    // per lane step.
+__global__ void __launch_bounds__(256) k_msm_hot_sum(MsmBatchDev b, const uint32_t* __restrict__ offs,
+                                                     const uint32_t* __restrict__ chunk2key, uint64_t stride,
+                                                     uint32_t* __restrict__ carry) {
+    using A = LanePoint<F>;
+    using S = LdsLanes<F, 256>;
+    __shared__ uint32_t shw[S::WORDS];
     __shared__ uint32_t hot[HOT_LIST];
     __shared__ uint64_t hbeg[HOT_LIST + 1];
     __shared__ uint64_t wmask[4];
     __shared__ uint32_t nhot;
+    __shared__ uint32_t seg_inst[256], seg_chunk[256], seg_cnt[256], nseg;
+    const S sh{shw};
+    // Most instances have no hot bucket. Each block lists the instances that
+    // do (largest bucket > HOT chunks), in instance order, with the prefix
+    // sums of their chunk counts, all in LDS; the grid then strides over the
+    // concatenated chunks of the hot instances only (over all chunks when the
+    // list overflows), 256 chunks at a time: each thread looks whether a
+    // segment starts at its chunk, then the whole block sums the found ones.
     const uint64_t* cbeg = space_g(b, SP_CHUNK);
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (threadIdx.x == 0) nhot = 0;
@@ -341,41 +340,64 @@ __global__ void __launch_bounds__(256) k_msm_hot_tree(MsmBatchDev b, const uint3
         __syncthreads();
     }
     const uint32_t nh = nhot;
-    const uint64_t step = (uint64_t)gridDim.x * blockDim.x;
-    if (nh > HOT_LIST) {   // more hot instances than the list holds: walk every chunk
-        for (uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; gid < cbeg[b.ninst]; gid += step) {
-            const uint32_t ii = find_inst_g(cbeg, b.ninst, gid);
-            if (b.stats[4 * ii + 2] > HOT * b.inst[ii].K)
-                hot_tree_chunk<F>(b, offs, chunk2key, stride, carry, ii, (uint32_t)(gid - cbeg[ii]));
-        }
-        return;
-    }
-    if (threadIdx.x == 0) {
+    if (nh == 0) return;
+    const bool listed = nh <= HOT_LIST;
+    if (listed && threadIdx.x == 0) {
         uint64_t t = 0;
         for (uint32_t h = 0; h < nh; ++h) { hbeg[h] = t; t += cbeg[hot[h] + 1] - cbeg[hot[h]]; }
         hbeg[nh] = t;
     }
     __syncthreads();
-    for (uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; g < hbeg[nh]; g += step) {
-        uint32_t lo = 0, hi = nh;   // hbeg[lo] <= g < hbeg[hi]
-        while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (hbeg[mid] <= g) lo = mid; else hi = mid;
+    const uint64_t total = listed ? hbeg[nh] : cbeg[b.ninst];
+    const uint32_t slot = threadIdx.x / A::LANES;
+    for (uint64_t base = (uint64_t)blockIdx.x * 256; base < total; base += (uint64_t)gridDim.x * 256) {
+        if (threadIdx.x == 0) nseg = 0;
+        __syncthreads();
+        const uint64_t g = base + threadIdx.x;
+        if (g < total) {
+            uint32_t ii, c;
+            if (listed) {
+                uint32_t lo = 0, hi = nh;   // hbeg[lo] <= g < hbeg[hi]
+                while (hi - lo > 1) {
+                    const uint32_t mid = (lo + hi) >> 1;
+                    if (hbeg[mid] <= g) lo = mid; else hi = mid;
+                }
+                ii = hot[lo], c = (uint32_t)(g - hbeg[lo]);
+            } else {
+                ii = find_inst_g(cbeg, b.ninst, g), c = (uint32_t)(g - cbeg[ii]);
+            }
+            const uint32_t cnt = hot_segment<F>(b, offs, chunk2key, stride, ii, c);
+            if (cnt > 1) {
+                const uint32_t at = atomicAdd(&nseg, 1u);
+                seg_inst[at] = ii, seg_chunk[at] = c, seg_cnt[at] = cnt;
+            }
         }
-        hot_tree_chunk<F>(b, offs, chunk2key, stride, carry, hot[lo], (uint32_t)(g - hbeg[lo]));
+        __syncthreads();
+        const uint32_t ns = nseg;
+        for (uint32_t q = 0; q < ns; ++q) {
+            const uint32_t cnt = seg_cnt[q];
+            uint32_t* first = carry + (size_t)A::RAW_WORDS * 2 * (cbeg[seg_inst[q]] + seg_chunk[q]);
+            const size_t step = (size_t)A::RAW_WORDS * 2 * stride;
+            A acc;
+            acc.set_inf();
+            for (uint32_t i = slot; i < cnt; i += S::SLOTS) acc.add(A::load_raw(first + step * i));
+            sh.tree_sum(acc, S::SLOTS);
+            if (slot == 0) acc.store_raw(first);
+        }
+        __syncthreads();
     }
 }
 
 // bucket spanning chunks f..l (f < l): bucket = tail(f) + heads(f+1..l), by
-// the lane of chunk f+1 (the first chunk that continues it)
+// the lane group of chunk f+1 (the first chunk that continues it)
 template <class F>
 __global__ void __launch_bounds__(256) k_msm_fixup(MsmBatchDev b, const uint32_t* __restrict__ offs,
-                                                   const uint32_t* __restrict__ chunk2key, const uint4* __restrict__ carry,
-                                                   uint4* __restrict__ bucket) {
-    using A = acc29_t<F>;
-    constexpr int RW = raw_vec<F>();
+                                                   const uint32_t* __restrict__ chunk2key, const uint32_t* __restrict__ carry,
+                                                   uint32_t* __restrict__ bucket) {
+    using A = LanePoint<F>;
+    constexpr int RW = A::RAW_WORDS;
     const uint64_t* cbeg = space_g(b, SP_CHUNK);
-    uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t gid = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / A::LANES;
     if (gid >= cbeg[b.ninst]) return;
     uint32_t ii = find_inst_g(cbeg, b.ninst, gid);
     const MsmInst& d = b.inst[ii];
@@ -387,58 +409,87 @@ __global__ void __launch_bounds__(256) k_msm_fixup(MsmBatchDev b, const uint32_t
     const uint32_t f = start / d.K;
     if (c != f + 1) return;
     const uint32_t l = (offs[kb + k + 1] - 1) / d.K;
-    const uint4* base = carry + (size_t)RW * 2 * cbeg[ii];
+    const uint32_t* base = carry + (size_t)RW * 2 * cbeg[ii];
     A acc = A::load_raw(base + (size_t)RW * (2 * f + 1));
-    if (l - f > HOT) {
-        acc.add(A::load_raw(base + (size_t)RW * 2 * (f + 1)));
-    } else {
-        for (uint32_t cc = f + 1; cc <= l; ++cc) acc.add(A::load_raw(base + (size_t)RW * 2 * cc));
-    }
+    const uint32_t last = l - f > HOT ? f + 1 : l;   // hot: their sum stands in the first
+    for (uint32_t cc = f + 1; cc <= last; ++cc) acc.add(A::load_raw(base + (size_t)RW * 2 * cc));
     acc.store_raw(bucket + (size_t)RW * (kb + k));
 }
 
 // ------------------------------------------------------------------ 7. bucket reduction
-// A window's value is sum_{d=1..NB} d * B_d. Bucket d = r*g + q + 1 lies in
-// run r (g buckets) at offset q, so the sum is
-//     sum_r [ A_r + g * r * R_r ],   A_r = sum_q (q+1) B,   R_r = sum_q B.
-// Stage 7a: lane per (window, run): A_r and R_r by running sums (2g
-// additions, no scalar multiplication). Stage 7b: workgroup per (window,
-// part of Gs = G/S runs): thread t takes m = Gs/T consecutive runs; the run
-// weights r become t*m + i inside the part, and sum_t t * rr_t (rr_t the
-// thread's run sum) is the sum over t >= 1 of the suffix sums of rr, one
-// LDS scan. Each part yields its value P_p (weights relative to the part's
-// first run) and its run sum RS_p; the host adds g * p * Gs * RS_p. Buckets,
-// run sums and the LDS slots hold raw accumulator states; only P_p and RS_p
-// are converted to R = 2^256 XYZZ points for the host.
-template <class F>
-__global__ void __launch_bounds__(128) k_bucket_segments(MsmBatchDev b, const uint4* __restrict__ bucket,
-                                                         const uint32_t* __restrict__ offs, uint4* __restrict__ segsum) {
-    using A = acc29_t<F>;
-    constexpr int RW = raw_vec<F>();
-    const uint64_t* rbeg = space_g(b, SP_BRED);
-    uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= rbeg[b.ninst]) return;
-    uint32_t ii = find_inst_g(rbeg, b.ninst, gid);
+// A window's value is sum_{d=1..NB} d * B_d. Workgroup per (window, part of
+// NB / S buckets), each lane group (slot) of it takes the g consecutive
+// buckets t*g .. t*g + g-1 of the part: with A_t = sum_q (q+1) B and R_t =
+// sum_q B by running sums (2g additions, no scalar multiplication) the part's
+// value, weights relative to its first bucket, is
+//     sum_t [ A_t + g * t * R_t ] = sum_t A_t + g * sum_{t>=1} X_t,
+// X_t the suffix sums of R, one LDS scan. Each part yields its value P_p and
+// its bucket sum RS_p; the host adds p * (NB / S) * RS_p. Buckets and LDS slots
+// hold raw accumulator states; only P_p and RS_p are converted to R = 2^256
+// XYZZ points for the host.
+// T = 256 threads for single MSMs, 64 in wide batches (fewer scan and tree
+// steps per bucket; the batch fills the GPU by itself).
+template <class F, int T>
+__global__ void __launch_bounds__(T) k_window_sum(MsmBatchDev b, const uint32_t* __restrict__ bucket, const uint32_t* __restrict__ offs,
+                                                  xyzz_t<F>* __restrict__ winsum) {
+    using A = LanePoint<F>;
+    using S = LdsLanes<F, T>;
+    constexpr int RW = A::RAW_WORDS;
+    __shared__ uint32_t shw[S::WORDS];
+    const S sh{shw};
+    const uint64_t* wbeg = space_g(b, SP_WIN);
+    const uint32_t ii = find_inst_g(wbeg, b.ninst, blockIdx.x);
     const MsmInst& d = b.inst[ii];
-    if (d.fused) return;   // its window-sum kernel reduces the runs itself
-    uint32_t t = (uint32_t)(gid - rbeg[ii]);
-    uint32_t j = t / d.G, sg = t % d.G;
-    const uint64_t kb = space_g(b, SP_KEY)[ii];
-    const uint32_t* of = offs + kb;
-    const uint4* bk = bucket + (size_t)RW * kb;
-    uint32_t kbase = j * d.NB + sg * d.g;
-    A run, acc;
+    const uint32_t local = (uint32_t)(blockIdx.x - wbeg[ii]);
+    const uint32_t j = local / d.S, part = local % d.S, PB = d.NB / d.S;   // buckets of the part
+    const uint32_t n = PB < (uint32_t)S::SLOTS ? PB : (uint32_t)S::SLOTS, m = PB / n;   // slots, buckets per slot
+    const uint32_t slot = threadIdx.x / A::LANES;
+    A a, run;
+    a.set_inf();
     run.set_inf();
-    acc.set_inf();
-    for (int q = (int)d.g - 1; q >= 0; --q) {
-        uint32_t key = kbase + q;
-        if (of[key + 1] != of[key]) run.add(A::load_raw(bk + (size_t)RW * key));
-        acc.add(run);
+    if (slot < n) {
+        const uint64_t kb = space_g(b, SP_KEY)[ii];
+        const uint32_t key0 = j * d.NB + part * PB + slot * m;
+        const uint32_t* of = offs + kb + key0;
+        const uint32_t* bk = bucket + (size_t)RW * (kb + key0);
+        auto load = [&](uint32_t q) {
+            A p;
+            if (of[q + 1] != of[q]) p = A::load_raw(bk + (size_t)RW * q);
+            else p.set_inf();
+            return p;
+        };
+        A next = load(m - 1);
+        for (int q = (int)m - 1; q >= 0; --q) {
+            run.add(next);
+            if (q > 0) next = load(q - 1);
+            a.add(run);
+        }
     }
-    acc.store_raw(segsum + (size_t)RW * 2 * gid);         // A_r
-    run.store_raw(segsum + (size_t)RW * (2 * gid + 1));   // R_r
+    // inclusive suffix scan of the slots' bucket sums
+    for (uint32_t off = 1; off < n; off <<= 1) {
+        __syncthreads();
+        sh.put(run);
+        __syncthreads();
+        if (slot + off < n) run.add(sh.get(off));
+    }
+    if (slot == 0) {
+        run.store_xyzz(winsum + 2 * blockIdx.x + 1);   // RS_p
+        run.set_inf();
+    }
+    for (uint32_t k = 1; k < m; k <<= 1) run.dbl();
+    a.add(run);
+    sh.tree_sum(a, n);
+    if (slot == 0) a.store_xyzz(winsum + 2 * blockIdx.x);   // P_p
 }
 
+// ------------------------------------------------------------------ 8. device-side combine (optional)
+// The host's combine as two kernels, in the 29-bit accumulator arithmetic.
+// k_msm_combine_windows: workgroup per (instance, window), lane per part p:
+// T_j = sum_p P_p + (g Gs) sum_p p RS_p, the last sum as the sum over p >= 1
+// of the suffix sums of RS (an LDS scan), stored as a raw state. k_msm_combine_horner: lane
+// per instance, Horner over the windows (the dependent doublings that make
+// this path slower than the host's), then the normalised Jacobian
+// (x, y, 1) or (0, 1, 0): the bytes the host writes.
 // Per-thread accumulator slots in LDS, word-major: word w of slot t at
 // sh[w * T + t], so the lanes of a wave touch consecutive words (a point per
 // slot in a row would put every lane's word w in the same bank)
@@ -474,106 +525,6 @@ HZK_DEV void lds_tree_sum(const LdsPoints<F, T>& sh, uint32_t t) {
     }
 }
 
-// T threads per part: 256 for single MSMs (shallow: the kernel is latency
-// bound there), 64 in wide batches (each thread takes 4x more runs, so the
-// scan and tree overhead per run is 4x smaller). Dynamic LDS: RAW_WORDS * T words.
-template <class F, int T>
-__global__ void __launch_bounds__(T) k_window_sum(MsmBatchDev b, const uint4* __restrict__ segsum,
-                                                  const uint4* __restrict__ bucket, const uint32_t* __restrict__ offs,
-                                                  xyzz_t<F>* __restrict__ winsum) {
-    using A = acc29_t<F>;
-    constexpr int RW = raw_vec<F>();
-    extern __shared__ uint32_t shw[];
-    const LdsPoints<F, T> sh{shw};
-    const uint64_t* wbeg = space_g(b, SP_WIN);
-    uint32_t ii = find_inst_g(wbeg, b.ninst, blockIdx.x);
-    const MsmInst& d = b.inst[ii];
-    const uint32_t local = (uint32_t)(blockIdx.x - wbeg[ii]);
-    const uint32_t j = local / d.S, part = local % d.S, Gs = d.G / d.S;
-    const uint32_t m = Gs >= T ? Gs / T : 1, t = threadIdx.x;
-    // runs t*m .. t*m + m - 1 of the part (A_r at 2r, R_r at 2r + 1)
-    const uint4* ss =
-        segsum + (size_t)RW * 2 * (space_g(b, SP_BRED)[ii] + (size_t)j * d.G + (size_t)part * Gs + (size_t)t * m);
-    A a, run, w;
-    a.set_inf();
-    run.set_inf();
-    w.set_inf();
-    if (d.fused) {
-        // m = 1: this lane's run r = part * T + t, buckets r*g .. r*g + g-1 of
-        // window j; A_r and R_r by running sums as in k_bucket_segments
-        const uint64_t kb = space_g(b, SP_KEY)[ii];
-        const uint32_t* of = offs + kb;
-        const uint4* bk = bucket + (size_t)RW * kb;
-        const uint32_t kbase = j * d.NB + (part * T + t) * d.g;
-        for (int q = (int)d.g - 1; q >= 0; --q) {
-            const uint32_t key = kbase + q;
-            if (of[key + 1] != of[key]) run.add(A::load_raw(bk + (size_t)RW * key));
-            a.add(run);
-        }
-    } else if (t * m < Gs) {
-        for (int i = (int)m - 1; i >= 0; --i) {
-            a.add(A::load_raw(ss + (size_t)RW * 2 * i));
-            run.add(A::load_raw(ss + (size_t)RW * (2 * i + 1)));
-            if (i > 0) w.add(run);   // w = sum_i i * R_i
-        }
-    }
-    // inclusive suffix scan of the thread run sums: slot t = sum_{t' >= t} rr_t'
-    sh.put(t, run);
-    __syncthreads();
-    for (uint32_t off = 1; off < T; off <<= 1) {
-        A x = sh.get(t);
-        if (t + off < T) x.add(sh.get(t + off));
-        __syncthreads();
-        sh.put(t, x);
-        __syncthreads();
-    }
-    const A part_sum = sh.get(0);
-    // P = sum_t a_t + g * sum_t (w_t + m * X_t), X_t = slot t for t >= 1
-    A u = sh.get(t);
-    if (t == 0) u.set_inf();
-    for (uint32_t k = 1; k < m; k <<= 1) u.dbl();
-    u.add(w);
-    if (T == 256) {
-        // shallow: the factor g per thread, one tree
-        for (uint32_t k = 1; k < d.g; k <<= 1) u.dbl();
-        u.add(a);
-        __syncthreads();
-        sh.put(t, u);
-        __syncthreads();
-        lds_tree_sum<F, T>(sh, t);
-        if (t == 0) {
-            winsum[2 * blockIdx.x] = sh.get(0).to_xyzz();   // P_p
-            winsum[2 * blockIdx.x + 1] = part_sum.to_xyzz();  // RS_p
-        }
-    } else {
-        // less work: both sums first, the factor g once
-        __syncthreads();
-        sh.put(t, u);
-        __syncthreads();
-        lds_tree_sum<F, T>(sh, t);
-        A total = sh.get(0);
-        __syncthreads();
-        sh.put(t, a);
-        __syncthreads();
-        lds_tree_sum<F, T>(sh, t);
-        if (t == 0) {
-            for (uint32_t k = 1; k < d.g; k <<= 1) total.dbl();
-            total.add(sh.get(0));
-            winsum[2 * blockIdx.x] = total.to_xyzz();         // P_p
-            winsum[2 * blockIdx.x + 1] = part_sum.to_xyzz();  // RS_p
-        }
-    }
-}
-
-// ------------------------------------------------------------------ 8. device-side combine (optional)
-// The host's combine as two kernels, in the 29-bit accumulator arithmetic.
-// k_msm_combine_windows: workgroup per (instance, window), lane per part p:
-// T_j = sum_p P_p + (g Gs) sum_p p RS_p, the last sum as the sum over p >= 1
-// of the suffix sums of RS (an LDS scan), stored as a raw state in the
-// run-sum area (free once the window sums exist). k_msm_combine_horner: lane
-// per instance, Horner over the windows (the dependent doublings that make
-// this path slower than the host's), then the normalised Jacobian
-// (x, y, 1) or (0, 1, 0): the bytes the host writes.
 template <class F>
 HZK_DEV acc29_t<F> acc_from_xyzz(const xyzz_t<F>& p);
 template <>
@@ -670,13 +621,13 @@ struct MsmBatchLayout {
     std::vector<uint64_t> begin;   // [SP_COUNT][ninst + 1]
     uint64_t tot[SP_COUNT];
     uint32_t max_nb = 1;
-    uint32_t tree_levels = 0;      // tree levels for hot buckets (upper bound)
+    uint32_t hot_levels = 0;       // levels of k_msm_hot_sum (upper bound)
     bool two_pass = false;         // some instance scatters in two passes
     int regime = 0;                // plan regime (MSM_REGIME_*)
     size_t bytes = 0;              // scratch needed
     // scratch offsets
     size_t o_inst, o_begin, o_stats, o_digits, o_hist, o_count, o_offs, o_tiles, o_sorted, o_coarse, o_chunk2key, o_bucket,
-        o_carry, o_segsum, o_win;
+        o_carry, o_tsum, o_win;
     // base arrays converted for the accumulation, one per distinct source
     // array (its largest referenced point count), and which one each instance reads
     std::vector<MsmConvTask> conv;     // dst holds the offset into the scratch until run time
@@ -743,15 +694,11 @@ static MsmBatchLayout msm_layout(hzk_ctx* ctx, const MsmJob* jobs, size_t count)
             d.T = T;
             d.tile = (d.n + T - 1) / T;
         }
-        d.S = 1;   // window-sum partials: at most ~2 run sums per lane of 256
-        while (d.S < 64 && d.G / d.S > 512) d.S *= 2;
-        // single MSMs: one run per lane of 256, reduced from the buckets inside
-        // the window-sum kernel (2g + 20 dependent additions per lane instead
-        // of 2g in a run-sum pass and then up to 28), while the W * G / 256
-        // workgroups of four waves fit one wave per SIMD (a second round of
-        // waves would double the kernel's latency-bound time)
-        d.fused = regime == MSM_REGIME_SINGLE && d.G % 256 == 0 && d.G / 256 <= 64 && (uint64_t)d.W * (d.G / 256) <= 256;
-        if (d.fused) d.S = d.G / 256;
+        // parts per window: one run of g buckets per slot of a window-sum
+        // workgroup, at most 64 parts (host combine, lanes of the device combine)
+        const uint32_t slots = regime == MSM_REGIME_BATCH ? LdsLanes<F, 64>::SLOTS : LdsLanes<F, 256>::SLOTS;
+        d.S = 1;
+        while (d.S < 64 && d.G / d.S > slots) d.S *= 2;
         uint64_t entries = (uint64_t)d.n * d.W;
         uint64_t sz[SP_COUNT];
         sz[SP_DIGIT] = d.nd;
@@ -759,7 +706,7 @@ static MsmBatchLayout msm_layout(hzk_ctx* ctx, const MsmJob* jobs, size_t count)
         sz[SP_KEY] = (uint64_t)d.nk + 1;
         sz[SP_SCANTILE] = ((uint64_t)d.nk + MSM_SCAN_TILE) / MSM_SCAN_TILE;
         sz[SP_CHUNK] = (entries + d.K - 1) / d.K;
-        sz[SP_BRED] = (uint64_t)d.W * d.G;
+        sz[SP_BRED] = (uint64_t)d.W;
         sz[SP_WIN] = (uint64_t)d.W * d.S;
         sz[SP_ENTRY] = (entries + 63) & ~(uint64_t)63;   // 256-B aligned per instance (vector index loads)
         sz[SP_HIST] = (uint64_t)d.T * d.nk;
@@ -770,8 +717,8 @@ static MsmBatchLayout msm_layout(hzk_ctx* ctx, const MsmJob* jobs, size_t count)
         uint64_t maxspan = (d.n + d.K - 1) / d.K + 1;   // a bucket holds at most n entries
         uint32_t lv = 0;
         if (maxspan > HOT)
-            for (uint64_t stride = 1; stride < maxspan; stride *= K2) ++lv;
-        if (lv > L.tree_levels) L.tree_levels = lv;
+            for (uint64_t stride = 1; stride < maxspan; stride *= hot_seg<F>()) ++lv;
+        if (lv > L.hot_levels) L.hot_levels = lv;
     }
     // two-pass scatter per instance, then the coarse-group space it needs
     uint64_t batch_entries = 0;
@@ -803,7 +750,7 @@ static MsmBatchLayout msm_layout(hzk_ctx* ctx, const MsmJob* jobs, size_t count)
     L.o_chunk2key = take(L.tot[SP_CHUNK] * 4);
     L.o_bucket = take(L.tot[SP_KEY] * raw);
     L.o_carry = take(2 * L.tot[SP_CHUNK] * raw);             // head and tail partial per chunk
-    L.o_segsum = take(2 * L.tot[SP_BRED] * raw);             // A_r, R_r per run
+    L.o_tsum = take(L.tot[SP_BRED] * raw);                   // window values (device-side combine)
     L.o_win = take(2 * L.tot[SP_WIN] * sizeof(xyzz_t<F>));   // P_p, RS_p per part (R = 2^256 points, for the host)
     {
         std::map<const void*, uint64_t> need;   // source array -> points referenced (virtual points of level tables)
@@ -847,7 +794,6 @@ static void msm_device_stages(hzk_ctx* ctx, const MsmBatchLayout& L, char* base)
     uint32_t* chunk2key = (uint32_t*)(base + L.o_chunk2key);
     uint4* bucket = (uint4*)(base + L.o_bucket);
     uint4* carry = (uint4*)(base + L.o_carry);
-    uint4* segsum = (uint4*)(base + L.o_segsum);
     xyzz_t<F>* win = (xyzz_t<F>*)(base + L.o_win);
     hipStream_t st = ctx->stream;
 
@@ -876,27 +822,21 @@ static void msm_device_stages(hzk_ctx* ctx, const MsmBatchLayout& L, char* base)
     }
     {
         TimedLaunch tl(ctx, "msm_fixup");
-        uint32_t stride = 1;
-        for (uint32_t lv = 0; lv < L.tree_levels; ++lv, stride *= K2)
-            hipLaunchKernelGGL(k_msm_hot_tree<F>, dim3(std::min<unsigned>(blocks_for(L.tot[SP_CHUNK], 256), 1024)), dim3(256), 0, st, b,
-                               (const uint32_t*)sb.offs, (const uint32_t*)chunk2key, stride, carry);
-        hipLaunchKernelGGL(k_msm_fixup<F>, dim3(blocks_for(L.tot[SP_CHUNK], 256)), dim3(256), 0, st, b, (const uint32_t*)sb.offs,
-                           (const uint32_t*)chunk2key, (const uint4*)carry, bucket);
+        uint64_t stride = 1;
+        for (uint32_t lv = 0; lv < L.hot_levels; ++lv, stride *= hot_seg<F>())
+            hipLaunchKernelGGL(k_msm_hot_sum<F>, dim3(std::min<unsigned>(blocks_for(L.tot[SP_CHUNK], 256), 1024)), dim3(256), 0, st, b,
+                               (const uint32_t*)sb.offs, (const uint32_t*)chunk2key, stride, (uint32_t*)carry);
+        hipLaunchKernelGGL(k_msm_fixup<F>, dim3(blocks_for(L.tot[SP_CHUNK] * LanePoint<F>::LANES, 256)), dim3(256), 0, st, b,
+                           (const uint32_t*)sb.offs, (const uint32_t*)chunk2key, (const uint32_t*)carry, (uint32_t*)bucket);
     }
     {
         TimedLaunch tl(ctx, "msm_bucket_reduce");
-        bool all_fused = true;
-        for (const MsmInst& d : L.inst) all_fused = all_fused && d.fused;
-        if (!all_fused)
-            hipLaunchKernelGGL(k_bucket_segments<F>, dim3(blocks_for(L.tot[SP_BRED], 128)), dim3(128), 0, st, b, (const uint4*)bucket,
-                               (const uint32_t*)sb.offs, segsum);
-        constexpr size_t WW = acc29_t<F>::RAW_WORDS * 4;   // LDS bytes per thread slot
         if (L.regime == MSM_REGIME_BATCH)
-            hipLaunchKernelGGL((k_window_sum<F, 64>), dim3((unsigned)L.tot[SP_WIN]), dim3(64), WW * 64, st, b, (const uint4*)segsum,
-                               (const uint4*)bucket, (const uint32_t*)sb.offs, win);
+            hipLaunchKernelGGL((k_window_sum<F, 64>), dim3((unsigned)L.tot[SP_WIN]), dim3(64), 0, st, b, (const uint32_t*)bucket,
+                               (const uint32_t*)sb.offs, win);
         else
-            hipLaunchKernelGGL((k_window_sum<F, 256>), dim3((unsigned)L.tot[SP_WIN]), dim3(256), WW * 256, st, b, (const uint4*)segsum,
-                               (const uint4*)bucket, (const uint32_t*)sb.offs, win);
+            hipLaunchKernelGGL((k_window_sum<F, 256>), dim3((unsigned)L.tot[SP_WIN]), dim3(256), 0, st, b, (const uint32_t*)bucket,
+                               (const uint32_t*)sb.offs, win);
     }
 }
 
@@ -909,7 +849,7 @@ static void msm_launch_combine(hzk_ctx* ctx, const MsmBatchLayout& L, char* base
     b.stats = (uint32_t*)(base + L.o_stats);
     uint32_t maxw = 1;
     for (const MsmInst& d : L.inst) maxw = std::max(maxw, d.W);
-    uint4* tsum = (uint4*)(base + L.o_segsum);   // W raw states per instance fit its run-sum range
+    uint4* tsum = (uint4*)(base + L.o_tsum);
     TimedLaunch tl(ctx, "msm_combine");
     hipLaunchKernelGGL(k_msm_combine_windows<F>, dim3((unsigned)(L.inst.size() * maxw)), dim3(64), 0, ctx->stream, b,
                        (const xyzz_t<F>*)(base + L.o_win), maxw, tsum);
@@ -955,9 +895,6 @@ int msm_batch_run(hzk_ctx* ctx, const MsmJob* jobs, size_t count, int dests_on_h
     for (size_t i = 0; i < count; ++i)   // bucket offsets are 32-bit
         HZK_CHECK(ctx, (uint64_t)L.inst[i].n * L.inst[i].W <= 0xffff0000ull, HZK_ERR_UNSUPPORTED,
                   "msm: n=%u with %u windows exceeds 2^32 bucket entries", L.inst[i].n, L.inst[i].W);
-    HZK_CHECK(ctx, (size_t)acc29_t<F>::RAW_WORDS * 4 * 256 <= ctx->lds_per_block, HZK_ERR_UNSUPPORTED,
-              "msm: the window sums need %zu B of LDS per workgroup, device allows %zu", (size_t)acc29_t<F>::RAW_WORDS * 4 * 256,
-              ctx->lds_per_block);
     HZK_CHECK(ctx, (size_t)L.max_nb * 4 <= ctx->lds_per_block, HZK_ERR_UNSUPPORTED,
               "msm: a %u-bucket window needs %u B of LDS per workgroup, device allows %zu", L.max_nb, L.max_nb * 4,
               ctx->lds_per_block);
