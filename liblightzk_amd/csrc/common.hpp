@@ -62,6 +62,10 @@ struct hzk_ctx {
     uint32_t last_msm[5] = {0, 0, 0, 0, 0};
     // NTT twiddle / coset tables for the last transform size (ntt.hip)
     void* ntt_cache = nullptr;
+    // workspace of transforms that permute on their last pass (ntt.hip): grown
+    // on demand in stream order, freed at destroy
+    void* ntt_ws = nullptr;
+    size_t ntt_ws_bytes = 0;
     // MSM plans [regime][G1, G2][log2 n]; regime 0: an MSM that has the GPU
     // to itself (latency), 1: an instance of a batch wide enough to fill the
     // GPU by itself (throughput)

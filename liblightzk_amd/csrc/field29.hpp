@@ -41,32 +41,12 @@ struct fq29 : limbs29 {
     static HZK_DEV fq29 unpack(const uint32_t* w) {
         return unpack(make_uint4(w[0], w[1], w[2], w[3]), make_uint4(w[4], w[5], w[6], w[7]));
     }
-    // the same from two 16-byte words (low, high) with no array in between:
-    // a small private array indexed in a loop can be placed in LDS by the
-    // compiler, which turns every base load into LDS traffic
-    static HZK_DEV fq29 unpack(const uint4& lo, const uint4& hi) {
-        fq29 r;
-        r.l[0] = lo.x & MASK;
-        r.l[1] = ((lo.x >> 29) | (lo.y << 3)) & MASK;
-        r.l[2] = ((lo.y >> 26) | (lo.z << 6)) & MASK;
-        r.l[3] = ((lo.z >> 23) | (lo.w << 9)) & MASK;
-        r.l[4] = ((lo.w >> 20) | (hi.x << 12)) & MASK;
-        r.l[5] = ((hi.x >> 17) | (hi.y << 15)) & MASK;
-        r.l[6] = ((hi.y >> 14) | (hi.z << 18)) & MASK;
-        r.l[7] = ((hi.z >> 11) | (hi.w << 21)) & MASK;
-        r.l[8] = hi.w >> 8;
-        return r;
-    }
+    static HZK_DEV fq29 unpack(const uint4& lo, const uint4& hi) { return limbs29::unpack(lo, hi); }
     // a canonical value back to 8 x 32-bit limbs
     HZK_DEV void pack(uint32_t* w) const {
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const int b = 32 * q, i = b / 29, s = b % 29;   // word q starts at bit s of limb i
-            uint64_t v = (uint64_t)(uint32_t)l[i] >> s;
-            v |= (uint64_t)(uint32_t)l[i + 1] << (29 - s);
-            if (i + 2 < 9 && 58 - s < 32) v |= (uint64_t)(uint32_t)l[i + 2] << (58 - s);
-            w[q] = (uint32_t)v;
-        }
+        uint4 lo, hi;
+        limbs29::pack(lo, hi);
+        w[0] = lo.x, w[1] = lo.y, w[2] = lo.z, w[3] = lo.w, w[4] = hi.x, w[5] = hi.y, w[6] = hi.z, w[7] = hi.w;
     }
     // y or p - y for y in [0, p], normalized
     static HZK_DEV fq29 negate_if(const fq29& y, bool neg) {

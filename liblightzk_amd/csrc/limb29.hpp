@@ -52,6 +52,15 @@ struct Fq29Mod {
                                        0x0ed815e2, 0x016626d2, 0x0b8bab0f, 0x0006d7c4};
 };
 
+struct Fr29Mod {
+    static constexpr uint32_t P[9] = {0x10000001, 0x1f0fac9f, 0x0e5c2450, 0x07d090f3, 0x1585d283,
+                                      0x02db40c0, 0x00a6e141, 0x0e5c2634, 0x0030644e};   // r
+    static constexpr uint32_t M0 = 0x0fffffff;     // -r^-1 mod 2^29
+    // (r M0 + 1) / 2^29
+    static constexpr uint32_t NP[9] = {0x18f05361, 0x012bb1fe, 0x0f5d8135, 0x1e6275f6, 0x07e7a880,
+                                       0x10c6bf1f, 0x11f74a6c, 0x06fdaecb, 0x00183227};
+};
+
 // acc += sum_i x[i] * y[i]: one v_mad_i64_i32 each, addend and sum in place.
 // As plain C++ the compiler re-associates a column into partial chains joined
 // by extra 64-bit adds. S: y are constants, held in scalar registers.
@@ -192,6 +201,30 @@ HZK_DEV void mad_one(int64_t& acc, int32_t x) { asm("v_mad_i64_i32 %0, vcc, %1, 
 struct limbs29 {
     int32_t l[9];
     static HZK_DEV limbs29 zero() { return {{0, 0, 0, 0, 0, 0, 0, 0, 0}}; }
+    // 8 x 32-bit limbs (a value < 2^256) from two 16-byte words (low, high); no
+    // array in between: a small private array indexed in a loop can be placed
+    // in LDS by the compiler
+    static HZK_DEV limbs29 unpack(const uint4& lo, const uint4& hi) {
+        limbs29 r;
+        r.l[0] = lo.x & MASK29;
+        r.l[1] = ((lo.x >> 29) | (lo.y << 3)) & MASK29;
+        r.l[2] = ((lo.y >> 26) | (lo.z << 6)) & MASK29;
+        r.l[3] = ((lo.z >> 23) | (lo.w << 9)) & MASK29;
+        r.l[4] = ((lo.w >> 20) | (hi.x << 12)) & MASK29;
+        r.l[5] = ((hi.x >> 17) | (hi.y << 15)) & MASK29;
+        r.l[6] = ((hi.y >> 14) | (hi.z << 18)) & MASK29;
+        r.l[7] = ((hi.z >> 11) | (hi.w << 21)) & MASK29;
+        r.l[8] = hi.w >> 8;
+        return r;
+    }
+    // a normalized value in [0, 2^256) back
+    HZK_DEV void pack(uint4& lo, uint4& hi) const {
+        uint32_t u[9];
+#pragma unroll
+        for (int i = 0; i < 9; ++i) u[i] = (uint32_t)l[i];
+        lo = make_uint4(u[0] | (u[1] << 29), (u[1] >> 3) | (u[2] << 26), (u[2] >> 6) | (u[3] << 23), (u[3] >> 9) | (u[4] << 20));
+        hi = make_uint4((u[4] >> 12) | (u[5] << 17), (u[5] >> 15) | (u[6] << 14), (u[6] >> 18) | (u[7] << 11), (u[7] >> 21) | (u[8] << 8));
+    }
     // limb by limb, no carries
     friend HZK_DEV limbs29 operator+(const limbs29& a, const limbs29& b) {
         limbs29 r;
