@@ -223,7 +223,6 @@ int hzk_ctx_create(int device, void* stream, hzk_ctx** out) {
     }
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, device) == hipSuccess) {
-        ctx->lds_per_block = prop.sharedMemPerBlock;
         ctx->num_cus = prop.multiProcessorCount;
     }
     if (stream) {

@@ -23,7 +23,6 @@ struct hzk_tune_entry {
 struct hzk_ctx {
     int device = 0;
     int num_cus = 256;
-    size_t lds_per_block = 65536;   // device limit, read at creation
     hipStream_t stream = nullptr;
     bool own_stream = false;
     std::string last_error;

@@ -466,8 +466,8 @@ int g16_msm_batch(hzk_ctx* ctx, G16Req* reqs, size_t n, int graph) {
     return rc;
 }
 
-// Upper bound of one MSM's scratch (digits and sorted entries, histograms,
-// key scans, bucket sums, chunk partials, window sums)
+// Upper bound of one MSM's scratch (digits, coarse and sorted entries, counts,
+// bucket sums, chunk partials, window sums)
 // for n points with xyzz points of pt_bytes (bucket sums and chunk partials
 // are raw 29-bit accumulator states, 9/8 of that), from the
 // built-in plans (the larger of the single-MSM and wide-batch regimes).
@@ -475,13 +475,11 @@ static size_t msm_scratch_bound(size_t n, size_t pt_bytes) {
     const size_t raw = pt_bytes / 8 * 9;
     size_t worst = 0;
     for (int regime : {MSM_REGIME_SINGLE, MSM_REGIME_BATCH}) {
-        const MsmPlan p = msm_plan_builtin(pt_bytes > 128, n, regime, 160 * 1024);
-        size_t W = p.W, nk = W * p.NB, entries = n * W;
-        size_t chunks = (entries + p.K - 1) / p.K;
-        const size_t coarse = p.NB >= 2048 && n >= MSM_TP_BATCH_MIN_N ? entries * 8 : 0;   // two-pass staging
-        size_t b = entries * 8 + coarse + (size_t)p.T * nk * 4 + 2 * (nk + 1) * 4 +
-                   2 * ((nk + 1 + MSM_SCAN_TILE) / MSM_SCAN_TILE) * 8 + (nk + 1) * raw + chunks * (4 + 2 * raw) +
-                   W * raw + 2 * 64 * W * pt_bytes + 4096;   // window values, part (P, RS) pairs
+        const MsmPlan p = msm_plan_builtin(pt_bytes > 128, n, regime);
+        const size_t W = p.W, nk = W * p.NB, entries = n * W, chunks = (entries + p.K - 1) / p.K;
+        const size_t cg = msm_coarse_groups(n, p.NB, p.W), groups = W * cg, pieces = entries / MSM_SUB + groups;
+        size_t b = entries * 14 + groups * msm_tiles(n) * 4 + pieces * (p.NB / cg) * 4 + (nk + 1) * 4 + (nk + 1) * raw +
+                   chunks * (4 + 2 * raw) + W * raw + 2 * 64 * W * pt_bytes + 65536;   // window values, part (P, RS) pairs
         worst = std::max(worst, b);
     }
     return worst;

@@ -4,28 +4,39 @@
 // Replaces the reference's operator (include/operator/msm.cuh:77-248: one
 // counting sort of n*win_cnt (bucket, point) pairs into 2^c buckets with
 // global atomics and a serial <<<1,1>>> scan, one 32-lane warp per bucket,
-// fixed <<<128,1024>>> geometry valid only for c = 12) with:
+// fixed <<<128,1024>>> geometry valid only for c = 12) with a two-level
+// counting sort per window (coarse groups of FB = NB / CG consecutive buckets,
+// then the buckets of each group):
 //
 //  1. recode   one lane per scalar: leave Montgomery form, signed c-bit digits
 //              d_j in [-2^(c-1), 2^(c-1)] over W = ceil(255/c) windows (the
 //              top window cannot carry because scalars are < r < 2^254),
 //              written window-major; digit 0 is dropped (the reference
-//              accumulates bucket 0 and scales it by 0, msm.cuh:121-161).
-//  2. histogram  one workgroup per (tile of scalars, window): counts in LDS
-//              (2^(c-1) counters, <= 128 KiB), one coalesced row per tile. No
-//              device-scope atomics: on a multi-XCD part they resolve past the
-//              per-XCD L2 and ran at ~5 G/s, slower than the whole accumulation.
-//  3. scan     per key a prefix over tiles, then an exclusive scan of the
-//              bucket counts -> bucket offsets; per-instance totals (entries,
-//              chunks, largest bucket) land in device stats, so no stage waits
-//              for the host.
-//  4. scatter  same (tile, window) workgroups: LDS cursors seeded from the
-//              scan, LDS atomics hand out slots, point index | sign<<31 is
-//              written into its bucket.
+//              accumulates bucket 0 and scales it by 0, msm.cuh:121-161). The
+//              workgroup counts its tile's digits by (window, coarse group) in
+//              LDS on the way.
+//  2. scan     exclusive scan of those counts in (window, group, tile) order:
+//              where every tile's entries of a group start; per group the
+//              pieces of MSM_SUB entries that the fine level works on.
+//  3. coarse scatter  workgroup per (tile, window): entries to their group,
+//              counting-sorted in LDS first so that consecutive lanes write
+//              consecutive addresses.
+//  4. fine level  workgroup per piece counts its entries by bucket, workgroup
+//              per group turns the counts into bucket offsets, workgroup per
+//              piece scatters. A group that one digit value fills (the ones of
+//              a witness) is many pieces, so no workgroup has more to do than
+//              the others; a histogram over all buckets of a window is never
+//              needed, so windows may have 2^19 buckets.
+//  1'-4'. instances of at most MSM_SMALL_N points with few buckets: the recode,
+//              then one workgroup per window sorts it whole in LDS.
 //  5-8 (msm_impl.hpp) chunked accumulation with boundary fix-up, bucket
 //              reduction, window sums;
 //  9. window combine on the host (Horner with c doublings per window) and
 //              normalisation; see host_ec.hpp for why this tail runs on the CPU.
+//
+// Per-instance totals (entries, chunks, largest bucket) land in device stats,
+// so no stage waits for the host. No device-scope atomics per entry: on a
+// multi-XCD part they resolve past the per-XCD L2 and ran at ~5 G/s.
 //
 // Every stage is one launch over the whole batch: each instance owns a
 // contiguous range of every work space (MsmSpace), and a lane finds its
@@ -41,7 +52,6 @@
 namespace hzk {
 
 static constexpr uint32_t DIGIT_NEG = 0x80000000u;
-static constexpr uint32_t MSM_MAX_FINE = (1u << (MSM_MAX_C - 1)) / MSM_COARSE;   // buckets per coarse group at most
 static constexpr int SCAN_ITEMS = 4;
 static constexpr int SCAN_THREADS = 256;
 static_assert(SCAN_ITEMS * SCAN_THREADS == MSM_SCAN_TILE, "scan tile");
@@ -57,190 +67,160 @@ HZK_DEV uint32_t find_inst(const uint64_t* __restrict__ beg, uint32_t ninst, uin
 }
 HZK_DEV const uint64_t* space(const MsmBatchDev& b, int s) { return b.begin + (size_t)s * (b.ninst + 1); }
 
+// exclusive scan of n LDS counters by a workgroup of T threads; returns the total
+template <int T>
+HZK_DEV uint32_t lds_exclusive_scan(const uint32_t* cnt, uint32_t* out, uint32_t* part, uint32_t n) {
+    const uint32_t t = threadIdx.x, per = (n + T - 1) / T, lo = min(n, t * per), hi = min(n, lo + per);
+    uint32_t s = 0;
+    for (uint32_t i = lo; i < hi; ++i) s += cnt[i];
+    // inclusive scan of the threads' sums: in the wave, then over the waves
+    uint32_t x = s;
+    for (uint32_t off = 1; off < 64; off <<= 1) {
+        const uint32_t y = __shfl_up(x, off, 64);
+        if ((t & 63) >= off) x += y;
+    }
+    if ((t & 63) == 63) part[t >> 6] = x;
+    __syncthreads();
+    uint32_t run = x - s, total = 0;
+    for (uint32_t w = 0; w < T / 64; ++w) {
+        if (w < (t >> 6)) run += part[w];
+        total += part[w];
+    }
+    for (uint32_t i = lo; i < hi; ++i) {
+        const uint32_t v = cnt[i];
+        out[i] = run;
+        run += v;
+    }
+    __syncthreads();
+    return total;
+}
+
 // ------------------------------------------------------------------ 1. digits
 // digits[j * n + i] = |d_ij| | sign << 31, or 0 for a zero digit. For a level
 // table of Lg levels the same array is, window by window of the pipeline, the
 // digits of Lg consecutive digit windows over nd * Lg virtual points
 // 2^(c (j mod Lg)) P_i, so Lg digit windows share one bucket set.
-__global__ void __launch_bounds__(256) k_msm_digits(MsmBatchDev b, uint32_t* __restrict__ digits) {
-    __shared__ uint32_t limbs[256][9];
-    const uint64_t* beg = space(b, SP_DIGIT);
-    const uint64_t* ebeg = space(b, SP_ENTRY);
-    const uint64_t total = beg[b.ninst];
-    for (uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; gid < total; gid += (uint64_t)gridDim.x * blockDim.x) {
-        uint32_t ii = find_inst(beg, b.ninst, gid);
-        const MsmInst& d = b.inst[ii];
-        uint32_t idx = (uint32_t)(gid - beg[ii]);
-        fr_t s = ((const fr_t*)d.scalars)[idx].from_mont();
-        uint32_t* my = limbs[threadIdx.x];
-        for (int w = 0; w < 8; ++w) my[w] = s.l[w];
-        my[8] = 0;
+// Workgroup per tile of scalars; its counts by (bucket set, coarse group) go
+// to count[(set * CG + group) * T + tile].
+// 1024 threads, or 256 where every tile of the launch is small (more
+// workgroups for a small MSM).
+__global__ void __launch_bounds__(1024) k_msm_digits(MsmBatchDev b, uint32_t* __restrict__ digits, uint32_t* __restrict__ count) {
+    extern __shared__ uint32_t cnt[];
+    const uint64_t* beg = space(b, SP_TILE);
+    const uint32_t ii = find_inst(beg, b.ninst, blockIdx.x);
+    const MsmInst& d = b.inst[ii];
+    // the instance's fields in registers: stores could alias them
+    const uint32_t t = (uint32_t)(blockIdx.x - beg[ii]), CG = d.CG, groups = d.W * CG, fshift = __ffs(d.FB) - 1;
+    const uint32_t nd = d.nd, Lg = d.Lg, Wd = d.Wd, windows = d.W * Lg, wb = d.wb, wx = d.wx;
+    const fr_t* scalars = (const fr_t*)d.scalars;
+    uint32_t* const dig = digits + space(b, SP_ENTRY)[ii];
+    for (uint32_t x = threadIdx.x; x < groups; x += blockDim.x) cnt[x] = 0;
+    if (t == 0 && threadIdx.x < 4) b.stats[4 * ii + threadIdx.x] = 0;
+    __syncthreads();
+    const uint32_t i1 = min(nd, (t + 1) * d.tile);
+    for (uint32_t idx = t * d.tile + threadIdx.x; idx < i1; idx += blockDim.x) {
+        fr_t s = scalars[idx].from_mont();
         uint32_t carry = 0;
-        uint32_t* out = digits + ebeg[ii] + idx;
-        // window j: bits [lo, lo + wj), wj = wb + 1 for j < wx, then wb (<= c);
-        // digits in [-2^(wj-1), 2^(wj-1)]
-        uint32_t lo = 0, wj = d.wb + (d.wx ? 1u : 0u);
+        uint32_t* out = dig + idx;
+        // window j: the next wj bits, wj = wb + 1 for j < wx, then wb (<= c);
+        // digits in [-2^(wj-1), 2^(wj-1)]. The scalar is shifted down in
+        // registers (words in LDS and two loads a window took 1.8 times as long)
+        uint32_t wj = wb + (wx ? 1u : 0u), level = 0, set = 0;
         uint32_t half = 1u << (wj - 1), mask = (1u << wj) - 1;
-        for (uint32_t j = 0; j < d.W * d.Lg; ++j) {   // level tables: windows past Wd pad the last set
+        for (uint32_t j = 0; j < windows; ++j) {   // level tables: windows past Wd pad the last set
             uint32_t dg = 0;
-            if (j == d.wx && d.wx) {
-                wj = d.wb;
+            if (j == wx && wx) {
+                wj = wb;
                 half = 1u << (wj - 1);
                 mask = (1u << wj) - 1;
             }
-            if (j < d.Wd) {
-                uint32_t w = lo >> 5, sh = lo & 31;
-                uint64_t v = (uint64_t)my[w] | ((uint64_t)my[w + 1] << 32);
-                uint32_t raw = ((uint32_t)(v >> sh) & mask) + carry;
+            if (j < Wd) {
+                const uint32_t raw = (s.l[0] & mask) + carry;
+#pragma unroll
+                for (int w = 0; w < 7; ++w) s.l[w] = __builtin_amdgcn_alignbit(s.l[w + 1], s.l[w], wj);
+                s.l[7] >>= wj;
                 if (raw > half) { carry = 1; dg = (2 * half - raw) | DIGIT_NEG; }
                 else { carry = 0; dg = raw; }
-                if ((dg & ~DIGIT_NEG) == 0) dg = 0;
-                lo += wj;
+                const uint32_t m = dg & ~DIGIT_NEG;
+                if (!m) dg = 0;
+                if (CG > 1) {
+                    if (m) atomicAdd(&cnt[set * CG + ((m - 1) >> fshift)], 1u);
+                } else {   // one counter per set: one addition per wave
+                    const uint64_t some = __ballot(m != 0);
+                    if (some && (threadIdx.x & 63) == (uint32_t)__builtin_ctzll(__ballot(1))) atomicAdd(&cnt[set], (uint32_t)__popcll(some));
+                }
             }
-            out[(size_t)j * d.nd] = dg;   // window j of scalar idx (level tables: set j / Lg, point (j % Lg) nd + idx)
+            out[(size_t)j * nd] = dg;   // window j of scalar idx (level tables: set j / Lg, point (j % Lg) nd + idx)
+            if (++level == Lg) level = 0, ++set;
         }
     }
-}
-
-// ------------------------------------------------------------------ 2. histogram
-// workgroup (t, j) of an instance counts the digits of scalars [t*tile, (t+1)*tile) in window j
-__global__ void __launch_bounds__(1024) k_msm_hist(MsmBatchDev b, const uint32_t* __restrict__ digits, uint32_t* __restrict__ hist) {
-    extern __shared__ uint32_t cnt[];
-    const uint64_t* beg = space(b, SP_TILEWG);
-    uint32_t ii = find_inst(beg, b.ninst, blockIdx.x);
-    const MsmInst& d = b.inst[ii];
-    uint32_t local = (uint32_t)(blockIdx.x - beg[ii]);
-    uint32_t t = local % d.T, j = local / d.T;
-    for (uint32_t x = threadIdx.x; x < d.NB; x += blockDim.x) cnt[x] = 0;
     __syncthreads();
-    const uint32_t i0 = t * d.tile, i1 = min(d.n, i0 + d.tile);
-    const size_t abs0 = space(b, SP_ENTRY)[ii] + (size_t)j * d.n;
-    const uint32_t* dj = digits + abs0;
-    auto count = [&](uint32_t dg) {
-        const uint32_t m = dg & ~DIGIT_NEG;
-        if (m) atomicAdd(&cnt[m - 1], 1u);
-    };
-    // 16-byte loads (four digits per lane) over the aligned middle of the
-    // tile, single digits for its at most 3 + 3 unaligned ends
-    uint32_t ia = i0 + ((4u - (uint32_t)((abs0 + i0) & 3)) & 3u);
-    if (ia > i1) ia = i1;
-    const uint32_t nv = (i1 - ia) / 4, ib = ia + 4 * nv;
-    for (uint32_t i = i0 + threadIdx.x; i < ia; i += blockDim.x) count(dj[i]);
-    for (uint32_t i = ib + threadIdx.x; i < i1; i += blockDim.x) count(dj[i]);
-    const uint4* dv = (const uint4*)(dj + ia);
-    for (uint32_t q = threadIdx.x; q < nv; q += blockDim.x) {
-        const uint4 w = dv[q];
-        count(w.x);
-        count(w.y);
-        count(w.z);
-        count(w.w);
-    }
-    __syncthreads();
-    uint32_t* row = hist + space(b, SP_HIST)[ii] + (size_t)t * d.nk + (size_t)j * d.NB;
-    for (uint32_t x = threadIdx.x; x < d.NB; x += blockDim.x) row[x] = cnt[x];
+    uint32_t* row = count + space(b, SP_CNT)[ii] + t;
+    for (uint32_t x = threadIdx.x; x < groups; x += blockDim.x) row[(size_t)x * d.T] = cnt[x];
 }
 
-// ------------------------------------------------------------------ 3. scans
-// per key: count = sum over tiles; hist[t][key] <- exclusive prefix over tiles
-__global__ void __launch_bounds__(256) k_msm_colscan(MsmBatchDev b, uint32_t* __restrict__ hist, uint32_t* __restrict__ count) {
-    const uint64_t* beg = space(b, SP_KEY);
-    uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= beg[b.ninst]) return;
-    uint32_t ii = find_inst(beg, b.ninst, gid);
-    const MsmInst& d = b.inst[ii];
-    uint32_t k = (uint32_t)(gid - beg[ii]);
-    if (k >= d.nk) { count[gid] = 0; return; }
-    uint32_t* h = hist + space(b, SP_HIST)[ii] + k;
-    uint32_t run = 0;
-    for (uint32_t t = 0; t < d.T; ++t) {
-        uint32_t v = h[(size_t)t * d.nk];
-        h[(size_t)t * d.nk] = run;
-        run += v;
-    }
-    count[gid] = run;
-}
-
-// one block per scan tile: tile sum and tile maximum
-__global__ void __launch_bounds__(SCAN_THREADS) k_scan_tiles(MsmBatchDev b, const uint32_t* __restrict__ count,
-                                                             uint64_t* __restrict__ tile_sum, uint64_t* __restrict__ tile_max) {
+// ------------------------------------------------------------------ 2. scans
+// exclusive scan, in place, of an instance's W * CG * T counts (and one more
+// place for the total). One block per scan tile: tile sum
+__global__ void __launch_bounds__(SCAN_THREADS) k_scan_tiles(MsmBatchDev b, const uint32_t* __restrict__ count, uint64_t* __restrict__ tile_sum) {
     __shared__ uint64_t red[SCAN_THREADS];
-    __shared__ uint32_t redmax[SCAN_THREADS];
     const uint64_t* tbeg = space(b, SP_SCANTILE);
     uint32_t ii = find_inst(tbeg, b.ninst, blockIdx.x);
     const MsmInst& d = b.inst[ii];
-    uint64_t kbase = space(b, SP_KEY)[ii];
-    uint32_t base = (uint32_t)(blockIdx.x - tbeg[ii]) * MSM_SCAN_TILE;
+    const uint64_t kbase = space(b, SP_CNT)[ii];
+    const uint32_t n = d.W * d.CG * d.T, base = (uint32_t)(blockIdx.x - tbeg[ii]) * MSM_SCAN_TILE;
     uint64_t s = 0;
-    uint32_t mx = 0;
     for (int t = 0; t < SCAN_ITEMS; ++t) {
         uint32_t k = base + threadIdx.x + t * SCAN_THREADS;
-        if (k <= d.nk) { uint32_t c = count[kbase + k]; s += c; mx = max(mx, c); }
+        if (k < n) s += count[kbase + k];
     }
     red[threadIdx.x] = s;
-    redmax[threadIdx.x] = mx;
     __syncthreads();
     for (int off = SCAN_THREADS / 2; off > 0; off >>= 1) {
-        if ((int)threadIdx.x < off) {
-            red[threadIdx.x] += red[threadIdx.x + off];
-            redmax[threadIdx.x] = max(redmax[threadIdx.x], redmax[threadIdx.x + off]);
-        }
+        if ((int)threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        tile_sum[blockIdx.x] = red[0];
-        tile_max[blockIdx.x] = redmax[0];
-    }
+    if (threadIdx.x == 0) tile_sum[blockIdx.x] = red[0];
 }
 
-// one block per instance: exclusive scan of its tile sums; totals to stats
-__global__ void __launch_bounds__(1024) k_scan_top(MsmBatchDev b, uint64_t* __restrict__ tile_sum, const uint64_t* __restrict__ tile_max) {
+// one block per instance: exclusive scan of its tile sums
+__global__ void __launch_bounds__(1024) k_scan_top(MsmBatchDev b, uint64_t* __restrict__ tile_sum) {
     __shared__ uint64_t part[1024];
-    __shared__ uint32_t pmax[1024];
     const uint64_t* tbeg = space(b, SP_SCANTILE);
     const uint32_t ii = blockIdx.x;
     const uint64_t t0 = tbeg[ii];
     const uint32_t ntiles = (uint32_t)(tbeg[ii + 1] - t0);
+    if (ntiles == 0) return;
     uint32_t per = (ntiles + 1023) / 1024;
-    uint32_t lo = threadIdx.x * per, hi = min(ntiles, lo + per);
+    uint32_t lo = min(ntiles, threadIdx.x * per), hi = min(ntiles, lo + per);
     uint64_t s = 0;
-    uint32_t mx = 0;
-    for (uint32_t i = lo; i < hi; ++i) { s += tile_sum[t0 + i]; mx = max(mx, (uint32_t)tile_max[t0 + i]); }
+    for (uint32_t i = lo; i < hi; ++i) s += tile_sum[t0 + i];
     part[threadIdx.x] = s;
-    pmax[threadIdx.x] = mx;
     __syncthreads();
     for (int off = 1; off < 1024; off <<= 1) {
         uint64_t v = (int)threadIdx.x >= off ? part[threadIdx.x - off] : 0;
-        uint32_t m = (int)threadIdx.x >= off ? pmax[threadIdx.x - off] : 0;
         __syncthreads();
         part[threadIdx.x] += v;
-        pmax[threadIdx.x] = max(pmax[threadIdx.x], m);
         __syncthreads();
     }
     uint64_t run = threadIdx.x ? part[threadIdx.x - 1] : 0;
     for (uint32_t i = lo; i < hi; ++i) { uint64_t v = tile_sum[t0 + i]; tile_sum[t0 + i] = run; run += v; }
-    if (threadIdx.x == 1023) {
-        const uint32_t entries = (uint32_t)part[1023], K = b.inst[ii].K;
-        b.stats[4 * ii + 0] = entries;
-        b.stats[4 * ii + 1] = (entries + K - 1) / K;
-        b.stats[4 * ii + 2] = pmax[1023];
-        b.stats[4 * ii + 3] = 0;
-    }
 }
 
-// per tile: exclusive scan -> bucket offsets for keys 0..nk
-__global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(MsmBatchDev b, const uint32_t* __restrict__ count,
-                                                             const uint64_t* __restrict__ tile_sum, uint32_t* __restrict__ offs) {
+// per tile: exclusive scan in place; place n takes the total
+__global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(MsmBatchDev b, uint32_t* __restrict__ count, const uint64_t* __restrict__ tile_sum) {
     __shared__ uint64_t part[SCAN_THREADS];
     const uint64_t* tbeg = space(b, SP_SCANTILE);
     uint32_t ii = find_inst(tbeg, b.ninst, blockIdx.x);
     const MsmInst& d = b.inst[ii];
-    uint64_t kbase = space(b, SP_KEY)[ii];
-    uint32_t base = (uint32_t)(blockIdx.x - tbeg[ii]) * MSM_SCAN_TILE + threadIdx.x * SCAN_ITEMS;
+    const uint64_t kbase = space(b, SP_CNT)[ii];
+    const uint32_t n = d.W * d.CG * d.T;
+    const uint32_t base = (uint32_t)(blockIdx.x - tbeg[ii]) * MSM_SCAN_TILE + threadIdx.x * SCAN_ITEMS;
     uint64_t v[SCAN_ITEMS];
     uint64_t s = 0;
     for (int t = 0; t < SCAN_ITEMS; ++t) {
         uint32_t k = base + t;
-        v[t] = k <= d.nk ? count[kbase + k] : 0;
+        v[t] = k < n ? count[kbase + k] : 0;
         s += v[t];
     }
     part[threadIdx.x] = s;
@@ -254,199 +234,327 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(MsmBatchDev b, cons
     uint64_t run = tile_sum[blockIdx.x] + (threadIdx.x ? part[threadIdx.x - 1] : 0);
     for (int t = 0; t < SCAN_ITEMS; ++t) {
         uint32_t k = base + t;
-        if (k <= d.nk) offs[kbase + k] = (uint32_t)run;
+        if (k <= n) count[kbase + k] = (uint32_t)run;
         run += v[t];
     }
 }
 
-// ------------------------------------------------------------------ 4. scatter
-__global__ void __launch_bounds__(1024) k_msm_scatter(MsmBatchDev b, const uint32_t* __restrict__ digits,
-                                                      const uint32_t* __restrict__ hist, const uint32_t* __restrict__ offs,
-                                                      uint32_t* __restrict__ sorted) {
-    extern __shared__ uint32_t cur[];
-    const uint64_t* beg = space(b, SP_TILEWG);
-    uint32_t ii = find_inst(beg, b.ninst, blockIdx.x);
+// one block per instance: pieces of each group, sub[g] = pieces before group
+// g, sub[W CG] = all; entry totals to stats
+__global__ void __launch_bounds__(1024) k_msm_pieces(MsmBatchDev b, const uint32_t* __restrict__ start, uint32_t* __restrict__ sub,
+                                                     uint32_t* __restrict__ offs) {
+    __shared__ uint32_t part[16];
+    const uint32_t ii = blockIdx.x;
     const MsmInst& d = b.inst[ii];
-    if (d.tp) return;   // scattered in two passes below
-    uint32_t local = (uint32_t)(blockIdx.x - beg[ii]);
-    uint32_t t = local % d.T, j = local / d.T;
-    const uint32_t* row = hist + space(b, SP_HIST)[ii] + (size_t)t * d.nk + (size_t)j * d.NB;
-    const uint32_t* of = offs + space(b, SP_KEY)[ii] + (size_t)j * d.NB;
-    for (uint32_t x = threadIdx.x; x < d.NB; x += blockDim.x) cur[x] = of[x] + row[x];
+    if (d.small) return;
+    const uint32_t groups = d.W * d.CG, per = (groups + 1023) / 1024, t = threadIdx.x;
+    const uint32_t* st = start + space(b, SP_CNT)[ii];
+    uint32_t* out = sub + space(b, SP_GROUP)[ii];
+    const uint32_t lo = min(groups, t * per), hi = min(groups, lo + per);
+    auto pieces = [&](uint32_t g) { return (st[(size_t)(g + 1) * d.T] - st[(size_t)g * d.T] + MSM_SUB - 1) / MSM_SUB; };
+    uint32_t s = 0;
+    for (uint32_t g = lo; g < hi; ++g) s += pieces(g);
+    uint32_t x = s;
+    for (uint32_t off = 1; off < 64; off <<= 1) {
+        const uint32_t y = __shfl_up(x, off, 64);
+        if ((t & 63) >= off) x += y;
+    }
+    if ((t & 63) == 63) part[t >> 6] = x;
     __syncthreads();
-    const uint32_t i0 = t * d.tile, i1 = min(d.n, i0 + d.tile);
-    const uint64_t ebase = space(b, SP_ENTRY)[ii];
-    const uint32_t* dj = digits + ebase + (size_t)j * d.n;
-    uint32_t* out = sorted + ebase;
-    for (uint32_t i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
-        uint32_t dg = dj[i];
-        uint32_t m = dg & ~DIGIT_NEG;
-        if (m) {
-            uint32_t pos = atomicAdd(&cur[m - 1], 1u);
-            out[pos] = i | (dg & DIGIT_NEG);
-        }
+    uint32_t run = x - s;
+    for (uint32_t w = 0; w < (t >> 6); ++w) run += part[w];
+    for (uint32_t g = lo; g < hi; ++g) {
+        out[g] = run;
+        run += pieces(g);
+    }
+    if (t == 1023) {
+        out[groups] = run;
+        const uint32_t entries = st[(size_t)groups * d.T];
+        b.stats[4 * ii + 0] = entries;
+        b.stats[4 * ii + 1] = (entries + d.K - 1) / d.K;
+        offs[space(b, SP_KEY)[ii] + d.nk] = entries;
     }
 }
 
-// ------------------------------------------------------------------ 4'. two-pass scatter
-// With 2^(c-1) >= 2048 buckets a single scatter writes each 4-byte entry to a
-// different bucket range: on the MI355X that became ~8x the entry bytes in HBM
-// writes (every write a separate partially-filled sector). The two passes
-// below write coalesced runs instead: pass 1 partitions each tile's entries by
-// coarse key (the top 8 bits of the bucket index, 256 groups per window) into
-// an 8-byte staging array laid out exactly like the final bucket ranges;
-// pass 2 sorts each coarse group by its low bits. In both, a round of
-// SC_ROUND entries is counting-sorted in LDS first, so consecutive lanes write
-// consecutive addresses of one group. 8192-entry rounds give a coarse group
-// about 32 entries (128 B) per round at 2^24 points; 4096 left half-filled
-// lines (2^24 MSM: both passes 2.18 ms with 4096, 1.84 ms with 8192, slower
-// again with 16384 and its single workgroup per CU).
+// ------------------------------------------------------------------ 3. coarse scatter
+// A round of SC_ROUND entries is counting-sorted in LDS first, so consecutive
+// lanes write consecutive addresses of one group. 8192-entry rounds give a
+// group of 256 about 32 entries (128 B) per round; 4096 left half-filled lines
+// (both levels of a 2^24 MSM 2.18 ms with 4096, 1.84 ms with 8192, slower again
+// with 16384 and its single workgroup per CU). An entry is its point index
+// (sign in bit 31) and its bucket within the group.
 static constexpr uint32_t SC_ROUND = 8192;
 static constexpr uint32_t SC_THREADS = 1024;
 static constexpr uint32_t SC_PER = SC_ROUND / SC_THREADS;
 static constexpr uint32_t SC_NONE = 0xffffffffu;
 
-// exclusive scan of n <= 1024 LDS counters (one thread per counter)
-HZK_DEV void lds_exclusive_scan(const uint32_t* cnt, uint32_t* out, uint32_t* tmp, uint32_t n) {
-    const uint32_t t = threadIdx.x;
-    if (t < n) tmp[t] = cnt[t];
-    __syncthreads();
-    for (uint32_t off = 1; off < n; off <<= 1) {
-        uint32_t v = (t < n && t >= off) ? tmp[t - off] : 0;
-        __syncthreads();
-        if (t < n) tmp[t] += v;
-        __syncthreads();
-    }
-    if (t < n) out[t] = tmp[t] - cnt[t];
-    __syncthreads();
-}
-
-// pass 1: workgroup per (tile, window) of a two-pass instance
 __global__ void __launch_bounds__(SC_THREADS) k_msm_scatter_coarse(MsmBatchDev b, const uint32_t* __restrict__ digits,
-                                                                   const uint32_t* __restrict__ hist, const uint32_t* __restrict__ offs,
-                                                                   uint2* __restrict__ coarse) {
-    __shared__ uint32_t cur[MSM_COARSE], cnt[MSM_COARSE], lstart[MSM_COARSE], tmp[MSM_COARSE];
-    __shared__ uint2 stage[SC_ROUND];
-    __shared__ uint8_t skey[SC_ROUND];
+                                                                   const uint32_t* __restrict__ start, uint32_t* __restrict__ cidx,
+                                                                   uint16_t* __restrict__ ckey) {
+    __shared__ uint32_t cur[MSM_MAX_COARSE], cnt[MSM_MAX_COARSE], lstart[MSM_MAX_COARSE], part[SC_THREADS / 64];
+    __shared__ uint32_t stage[SC_ROUND], skey[SC_ROUND];
     const uint64_t* beg = space(b, SP_TILEWG);
     const uint32_t ii = find_inst(beg, b.ninst, blockIdx.x);
     const MsmInst& d = b.inst[ii];
-    if (!d.tp) return;
     const uint32_t local = (uint32_t)(blockIdx.x - beg[ii]);
-    const uint32_t t = local % d.T, j = local / d.T;
-    const uint32_t FB = d.NB / MSM_COARSE, fshift = __ffs(FB) - 1;
+    // the instance's fields in registers: stores could alias them
+    const uint32_t T = d.T, ctile = d.ctile, CG = d.CG, fmask = d.FB - 1, fshift = __ffs(d.FB) - 1, ib = d.ib, nd = d.nd, Lg = d.Lg, n = d.n;
+    const uint32_t per = (T + ctile - 1) / ctile;   // workgroups per window, ctile tiles each
+    const uint32_t t = (local % per) * ctile, j = local / per;
     const uint32_t tid = threadIdx.x;
-    // cursor of coarse group h: start of its first bucket + this tile's prefix over its buckets
-    if (tid < MSM_COARSE) {
-        const uint32_t* row = hist + space(b, SP_HIST)[ii] + (size_t)t * d.nk + (size_t)j * d.NB + (size_t)tid * FB;
-        uint32_t acc = offs[space(b, SP_KEY)[ii] + (size_t)j * d.NB + (size_t)tid * FB];
-        for (uint32_t q = 0; q < FB; ++q) acc += row[q];
-        cur[tid] = acc;
-    }
-    const uint32_t i0 = t * d.tile, i1 = min(d.n, i0 + d.tile);
+    const uint32_t* st = start + space(b, SP_CNT)[ii] + (size_t)j * CG * T + t;
+    for (uint32_t h = tid; h < CG; h += SC_THREADS) cur[h] = st[(size_t)h * T];
+    const uint32_t i0 = min(nd, t * d.tile), i1 = min(nd, i0 + ctile * d.tile);
     const uint64_t ebase = space(b, SP_ENTRY)[ii];
-    const uint32_t* dj = digits + ebase + (size_t)j * d.n;
-    uint2* out = coarse + ebase;
-    for (uint32_t base = i0; base < i1; base += SC_ROUND) {
-        if (tid < MSM_COARSE) cnt[tid] = 0;
-        __syncthreads();
-        uint32_t val[SC_PER], key[SC_PER], rank[SC_PER];
-        for (uint32_t k = 0; k < SC_PER; ++k) {
-            const uint32_t i = base + tid + k * SC_THREADS;
-            rank[k] = SC_NONE;
-            if (i < i1) {
-                const uint32_t dg = dj[i], m = dg & ~DIGIT_NEG;
-                if (m) {
-                    key[k] = m - 1;
-                    val[k] = i | (dg & DIGIT_NEG);
-                    rank[k] = atomicAdd(&cnt[(m - 1) >> fshift], 1u);
-                }
+    uint32_t* oi = cidx + ebase;
+    uint16_t* ok = ckey + ebase;
+    for (uint32_t level = 0; level < Lg; ++level) {
+        const uint32_t first = level * nd;
+        const uint32_t* dj = digits + ebase + (size_t)j * n + first;
+        for (uint32_t base = i0; base < i1; base += SC_ROUND) {
+            for (uint32_t h = tid; h < CG; h += SC_THREADS) cnt[h] = 0;
+            __syncthreads();
+            uint32_t dg[SC_PER], key[SC_PER], rank[SC_PER];
+#pragma unroll
+            for (uint32_t k = 0; k < SC_PER; ++k) {   // all loads before the first use
+                const uint32_t i = base + tid + k * SC_THREADS;
+                dg[k] = i < i1 ? dj[i] : 0;
             }
-        }
-        __syncthreads();
-        lds_exclusive_scan(cnt, lstart, tmp, MSM_COARSE);
-        for (uint32_t k = 0; k < SC_PER; ++k) {
-            if (rank[k] == SC_NONE) continue;
-            const uint32_t h = key[k] >> fshift, p = lstart[h] + rank[k];
-            stage[p] = make_uint2(val[k], key[k] & (FB - 1));
-            skey[p] = (uint8_t)h;
-        }
-        __syncthreads();
-        const uint32_t total = lstart[MSM_COARSE - 1] + cnt[MSM_COARSE - 1];
-        if (d.tp == 2) {   // packed: point index < 2^24 and fine key < 128 share one word with the sign
-            uint32_t* out32 = (uint32_t*)out;
+#pragma unroll
+            for (uint32_t k = 0; k < SC_PER; ++k) {
+                key[k] = (dg[k] & ~DIGIT_NEG) - 1;
+                rank[k] = dg[k] ? atomicAdd(&cnt[key[k] >> fshift], 1u) : SC_NONE;
+            }
+            __syncthreads();
+            const uint32_t total = lds_exclusive_scan<SC_THREADS>(cnt, lstart, part, CG);
+#pragma unroll
+            for (uint32_t k = 0; k < SC_PER; ++k) {
+                if (rank[k] == SC_NONE) continue;
+                const uint32_t p = lstart[key[k] >> fshift] + rank[k];
+                const uint32_t val = (first + base + tid + k * SC_THREADS) | (dg[k] & DIGIT_NEG);
+                stage[p] = ib ? val | ((key[k] & fmask) << ib) : val;
+                skey[p] = key[k];
+            }
+            __syncthreads();
             for (uint32_t p = tid; p < total; p += SC_THREADS) {
-                const uint32_t h = skey[p];
-                out32[cur[h] + (p - lstart[h])] = stage[p].x | (stage[p].y << 24);
+                const uint32_t key2 = skey[p], h = key2 >> fshift, to = cur[h] + (p - lstart[h]);
+                oi[to] = stage[p];
+                if (!ib) ok[to] = (uint16_t)(key2 & fmask);
             }
-        } else {
-            for (uint32_t p = tid; p < total; p += SC_THREADS) {
-                const uint32_t h = skey[p];
-                out[cur[h] + (p - lstart[h])] = stage[p];
-            }
+            __syncthreads();
+            for (uint32_t h = tid; h < CG; h += SC_THREADS) cur[h] += cnt[h];
+            __syncthreads();
         }
-        __syncthreads();
-        if (tid < MSM_COARSE) cur[tid] += cnt[tid];
-        __syncthreads();
     }
 }
 
-// pass 2: workgroup per (window, coarse group): bucket order inside the group
-__global__ void __launch_bounds__(SC_THREADS) k_msm_scatter_fine(MsmBatchDev b, const uint2* __restrict__ coarse,
-                                                                 const uint32_t* __restrict__ offs, uint32_t* __restrict__ sorted) {
-    __shared__ uint32_t cur[MSM_MAX_FINE], cnt[MSM_MAX_FINE], lstart[MSM_MAX_FINE], tmp[MSM_MAX_FINE];
-    __shared__ uint32_t stage[SC_ROUND];
-    __shared__ uint8_t skey[SC_ROUND];
-    const uint64_t* beg = space(b, SP_CGROUP);
+// ------------------------------------------------------------------ 4. fine level
+struct MsmPiece { uint32_t group, e0, e1; };   // entries [e0, e1) of a group
+// the piece of an instance's local piece number, or group = UINT32_MAX past the last
+HZK_DEV MsmPiece find_piece(const MsmInst& d, const uint32_t* __restrict__ sub, const uint32_t* __restrict__ start, uint32_t local) {
+    uint32_t lo = 0, hi = d.W * d.CG;
+    if (local >= sub[hi]) return {UINT32_MAX, 0, 0};
+    while (hi - lo > 1) {   // sub[lo] <= local < sub[hi]; empty groups are skipped by taking the last such lo
+        const uint32_t mid = (lo + hi) >> 1;
+        if (sub[mid] <= local) lo = mid; else hi = mid;
+    }
+    const uint32_t g0 = start[(size_t)lo * d.T], g1 = start[(size_t)(lo + 1) * d.T], e0 = g0 + (local - sub[lo]) * MSM_SUB;
+    return {lo, e0, min(g1, e0 + MSM_SUB)};
+}
+
+// workgroup per piece: counts by bucket of the group
+__global__ void __launch_bounds__(512) k_msm_fine_count(MsmBatchDev b, const uint32_t* __restrict__ start, const uint32_t* __restrict__ sub,
+                                                        const uint32_t* __restrict__ cidx, const uint16_t* __restrict__ ckey,
+                                                        uint32_t* __restrict__ rows) {
+    extern __shared__ uint32_t dyn[];
+    const uint64_t* beg = space(b, SP_SUB);
     const uint32_t ii = find_inst(beg, b.ninst, blockIdx.x);
     const MsmInst& d = b.inst[ii];
-    if (!d.tp) return;
     const uint32_t local = (uint32_t)(blockIdx.x - beg[ii]);
-    const uint32_t FB = d.NB / MSM_COARSE;
-    const uint32_t* of = offs + space(b, SP_KEY)[ii] + (size_t)local * FB;   // local = j * 256 + h
-    const uint32_t tid = threadIdx.x;
-    const uint32_t g0 = of[0], g1 = of[FB];
-    if (tid < FB) cur[tid] = of[tid];
-    const uint64_t ebase = space(b, SP_ENTRY)[ii];
-    const uint2* in = coarse + ebase;
-    const uint32_t* in32 = (const uint32_t*)in;   // packed entries (tp == 2)
-    const bool packed = d.tp == 2;
-    uint32_t* out = sorted + ebase;
-    for (uint32_t base = g0; base < g1; base += SC_ROUND) {
-        if (tid < FB) cnt[tid] = 0;
-        __syncthreads();
-        uint2 v[SC_PER];
-        uint32_t rank[SC_PER];
-        for (uint32_t k = 0; k < SC_PER; ++k) {
-            const uint32_t e = base + tid + k * SC_THREADS;
-            rank[k] = SC_NONE;
-            if (e < g1) {
-                if (packed) {
-                    const uint32_t w = in32[e];
-                    v[k] = make_uint2(w & 0x80ffffffu, (w >> 24) & 0x7fu);
-                } else {
-                    v[k] = in[e];
-                }
-                rank[k] = atomicAdd(&cnt[v[k].y], 1u);
-            }
+    const MsmPiece p = find_piece(d, sub + space(b, SP_GROUP)[ii], start + space(b, SP_CNT)[ii], local);
+    if (p.group == UINT32_MAX) return;
+    for (uint32_t f = threadIdx.x; f < d.FB; f += 512) dyn[f] = 0;
+    __syncthreads();
+    const uint64_t ebase = space(b, SP_ENTRY)[ii];   // a multiple of 64 entries
+    const uint32_t ib = d.ib, fmask = d.FB - 1;
+    if (ib) {
+        // 16-byte loads over the aligned middle, single entries at the ends
+        const uint32_t* in = cidx + ebase;
+        auto count = [&](uint32_t w) { atomicAdd(&dyn[(w >> ib) & fmask], 1u); };
+        const uint32_t ea = min(p.e1, (p.e0 + 3) & ~3u), nv = (p.e1 - ea) / 4, eb = ea + 4 * nv;
+        if (p.e0 + threadIdx.x < ea) count(in[p.e0 + threadIdx.x]);
+        if (eb + threadIdx.x < p.e1) count(in[eb + threadIdx.x]);
+        const uint4* in4 = (const uint4*)(in + ea);
+        for (uint32_t q = threadIdx.x; q < nv; q += 512) {
+            const uint4 w = in4[q];
+            count(w.x);
+            count(w.y);
+            count(w.z);
+            count(w.w);
         }
+    } else {
+        const uint16_t* key = ckey + ebase;
+        for (uint32_t e = p.e0 + threadIdx.x; e < p.e1; e += 512) atomicAdd(&dyn[key[e]], 1u);
+    }
+    __syncthreads();
+    uint32_t* row = rows + space(b, SP_ROW)[ii] + (size_t)local * d.FB;
+    for (uint32_t f = threadIdx.x; f < d.FB; f += 512) row[f] = dyn[f];
+}
+
+// workgroup per group: bucket offsets; the pieces' counts become where each
+// piece's entries of a bucket start
+__global__ void __launch_bounds__(256) k_msm_fine_offsets(MsmBatchDev b, const uint32_t* __restrict__ start, const uint32_t* __restrict__ sub,
+                                                          uint32_t* __restrict__ rows, uint32_t* __restrict__ offs) {
+    extern __shared__ uint32_t dyn[];   // FB totals, FB starts
+    __shared__ uint32_t part[4], mx;
+    const uint64_t* beg = space(b, SP_GROUP);
+    const uint32_t ii = find_inst(beg, b.ninst, blockIdx.x);
+    const MsmInst& d = b.inst[ii];
+    const uint32_t g = (uint32_t)(blockIdx.x - beg[ii]);
+    if (d.small || g >= d.W * d.CG) return;
+    const uint32_t* su = sub + beg[ii];
+    const uint32_t s0 = su[g], s1 = su[g + 1], g0 = start[space(b, SP_CNT)[ii] + (size_t)g * d.T];
+    uint32_t* row = rows + space(b, SP_ROW)[ii];
+    uint32_t *tot = dyn, *at = dyn + d.FB;
+    uint32_t largest = 0;
+    if (threadIdx.x == 0) mx = 0;
+    for (uint32_t f = threadIdx.x; f < d.FB; f += 256) {
+        uint32_t s = 0;
+        for (uint32_t q = s0; q < s1; ++q) s += row[(size_t)q * d.FB + f];
+        tot[f] = s;
+        largest = max(largest, s);
+    }
+    __syncthreads();
+    lds_exclusive_scan<256>(tot, at, part, d.FB);
+    atomicMax(&mx, largest);
+    uint32_t* of = offs + space(b, SP_KEY)[ii] + (size_t)g * d.FB;   // g = window * CG + group
+    for (uint32_t f = threadIdx.x; f < d.FB; f += 256) {
+        uint32_t run = g0 + at[f];
+        of[f] = run;
+        for (uint32_t q = s0; q < s1; ++q) {
+            const uint32_t v = row[(size_t)q * d.FB + f];
+            row[(size_t)q * d.FB + f] = run;
+            run += v;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && mx) atomicMax(&b.stats[4 * ii + 2], mx);
+}
+
+// workgroup per piece: entries to their bucket, staged in LDS as in the coarse scatter
+__global__ void __launch_bounds__(SC_THREADS) k_msm_scatter_fine(MsmBatchDev b, const uint32_t* __restrict__ start,
+                                                                 const uint32_t* __restrict__ sub, const uint32_t* __restrict__ rows,
+                                                                 const uint32_t* __restrict__ cidx, const uint16_t* __restrict__ ckey,
+                                                                 uint32_t* __restrict__ sorted) {
+    extern __shared__ uint32_t dyn[];   // per bucket of the group: cursor, count, start in the round
+    __shared__ uint32_t stage[SC_ROUND], part[SC_THREADS / 64];
+    __shared__ uint16_t skey[SC_ROUND];
+    const uint64_t* beg = space(b, SP_SUB);
+    const uint32_t ii = find_inst(beg, b.ninst, blockIdx.x);
+    const MsmInst& d = b.inst[ii];
+    const uint32_t local = (uint32_t)(blockIdx.x - beg[ii]);
+    const MsmPiece pc = find_piece(d, sub + space(b, SP_GROUP)[ii], start + space(b, SP_CNT)[ii], local);
+    if (pc.group == UINT32_MAX) return;
+    const uint32_t FB = d.FB, ib = d.ib, tid = threadIdx.x;
+    uint32_t *cur = dyn, *cnt = dyn + FB, *lstart = dyn + 2 * FB;
+    const uint32_t* row = rows + space(b, SP_ROW)[ii] + (size_t)local * FB;
+    for (uint32_t f = tid; f < FB; f += SC_THREADS) cur[f] = row[f];
+    const uint64_t ebase = space(b, SP_ENTRY)[ii];
+    const uint32_t* in = cidx + ebase;
+    const uint16_t* ik = ckey + ebase;
+    uint32_t* out = sorted + ebase;
+    for (uint32_t base = pc.e0; base < pc.e1; base += SC_ROUND) {
+        for (uint32_t f = tid; f < FB; f += SC_THREADS) cnt[f] = 0;
         __syncthreads();
-        lds_exclusive_scan(cnt, lstart, tmp, FB);
+        uint32_t v[SC_PER], key[SC_PER], rank[SC_PER];
+        const uint32_t e0 = base + tid, e1 = pc.e1;
+#pragma unroll
+        for (uint32_t k = 0; k < SC_PER; ++k) v[k] = e0 + k * SC_THREADS < e1 ? in[e0 + k * SC_THREADS] : 0;   // all loads before the first use
+        if (ib) {
+#pragma unroll
+            for (uint32_t k = 0; k < SC_PER; ++k) {
+                key[k] = (v[k] >> ib) & (FB - 1);
+                v[k] &= 0x80000000u | ((1u << ib) - 1);
+            }
+        } else {
+#pragma unroll
+            for (uint32_t k = 0; k < SC_PER; ++k) key[k] = e0 + k * SC_THREADS < e1 ? ik[e0 + k * SC_THREADS] : 0;
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < SC_PER; ++k) rank[k] = e0 + k * SC_THREADS < e1 ? atomicAdd(&cnt[key[k]], 1u) : SC_NONE;
+        __syncthreads();
+        const uint32_t total = lds_exclusive_scan<SC_THREADS>(cnt, lstart, part, FB);
+#pragma unroll
         for (uint32_t k = 0; k < SC_PER; ++k) {
             if (rank[k] == SC_NONE) continue;
-            const uint32_t p = lstart[v[k].y] + rank[k];
-            stage[p] = v[k].x;
-            skey[p] = (uint8_t)v[k].y;
+            const uint32_t p = lstart[key[k]] + rank[k];
+            stage[p] = v[k];
+            skey[p] = (uint16_t)key[k];
         }
         __syncthreads();
-        const uint32_t total = min(SC_ROUND, g1 - base);
         for (uint32_t p = tid; p < total; p += SC_THREADS) {
             const uint32_t f = skey[p];
             out[cur[f] + (p - lstart[f])] = stage[p];
         }
         __syncthreads();
-        if (tid < FB) cur[tid] += cnt[tid];
+        for (uint32_t f = tid; f < FB; f += SC_THREADS) cur[f] += cnt[f];
         __syncthreads();
+    }
+}
+
+// ------------------------------------------------------------------ 4'. small instances
+// workgroup per bucket set: counts, offsets and order in LDS; count holds the
+// recode's entries per (set, tile)
+__global__ void __launch_bounds__(1024) k_msm_sort_small(MsmBatchDev b, const uint32_t* __restrict__ digits, const uint32_t* __restrict__ count,
+                                                         uint32_t* __restrict__ offs, uint32_t* __restrict__ sorted) {
+    extern __shared__ uint32_t dyn[];   // NB counts, NB cursors
+    __shared__ uint32_t part[16], before, all, mx;
+    const uint64_t* beg = space(b, SP_SMALL);
+    const uint32_t ii = find_inst(beg, b.ninst, blockIdx.x);
+    const MsmInst& d = b.inst[ii];
+    const uint32_t j = (uint32_t)(blockIdx.x - beg[ii]), tid = threadIdx.x, n = d.n;
+    uint32_t *cnt = dyn, *cur = dyn + d.NB;
+    for (uint32_t x = tid; x < d.NB; x += 1024) cnt[x] = 0;
+    if (tid == 0) before = all = mx = 0;
+    __syncthreads();
+    const uint32_t* ct = count + space(b, SP_CNT)[ii];
+    uint32_t s0 = 0, s1 = 0;
+    for (uint32_t q = tid; q < d.W * d.T; q += 1024) {
+        const uint32_t v = ct[q];
+        s1 += v;
+        if (q < j * d.T) s0 += v;
+    }
+    if (s1) atomicAdd(&all, s1);
+    if (s0) atomicAdd(&before, s0);
+    const uint64_t ebase = space(b, SP_ENTRY)[ii];
+    const uint32_t* dj = digits + ebase + (size_t)j * n;
+    for (uint32_t i = tid; i < n; i += 1024) {
+        const uint32_t m = dj[i] & ~DIGIT_NEG;
+        if (m) atomicAdd(&cnt[m - 1], 1u);
+    }
+    __syncthreads();
+    lds_exclusive_scan<1024>(cnt, cur, part, d.NB);
+    uint32_t* of = offs + space(b, SP_KEY)[ii] + (size_t)j * d.NB;
+    uint32_t largest = 0;
+    for (uint32_t x = tid; x < d.NB; x += 1024) {
+        cur[x] += before;
+        of[x] = cur[x];
+        largest = max(largest, cnt[x]);
+    }
+    if (largest) atomicMax(&mx, largest);
+    __syncthreads();
+    if (tid == 0) {
+        if (mx) atomicMax(&b.stats[4 * ii + 2], mx);
+        if (j + 1 == d.W) {
+            of[d.NB] = all;
+            b.stats[4 * ii + 0] = all;
+            b.stats[4 * ii + 1] = (all + d.K - 1) / d.K;
+        }
+    }
+    uint32_t* out = sorted + ebase;
+    for (uint32_t i = tid; i < n; i += 1024) {
+        const uint32_t dg = dj[i], m = dg & ~DIGIT_NEG;
+        if (m) out[atomicAdd(&cur[m - 1], 1u)] = i | (dg & DIGIT_NEG);
     }
 }
 
@@ -454,63 +562,53 @@ __global__ void __launch_bounds__(SC_THREADS) k_msm_scatter_fine(MsmBatchDev b, 
 void msm_prepare() {
     static std::once_flag once;
     std::call_once(once, [] {
-        int bytes = (1 << (MSM_MAX_C - 1)) * 4;
-        (void)hipFuncSetAttribute((const void*)k_msm_hist, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-        (void)hipFuncSetAttribute((const void*)k_msm_scatter, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+        auto allow = [](const void* k, size_t bytes) { (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes); };
+        allow((const void*)k_msm_scatter_fine, 12 * MSM_MAX_FINE);
+        allow((const void*)k_msm_sort_small, 8 * MSM_SMALL_NB);
     });
 }
 
-static unsigned grid_for(uint64_t n, unsigned threads, unsigned cap) {
-    uint64_t g = (n + threads - 1) / threads;
-    if (g < 1) g = 1;
-    return (unsigned)(g < cap ? g : cap);
-}
-
-void msm_launch_scalar_stages(hzk_ctx* ctx, const MsmBatchDev& b, const uint64_t* tot, uint32_t max_nb,
-                              const MsmScalarBufs& bufs) {
+void msm_launch_scalar_stages(hzk_ctx* ctx, const MsmBatchDev& b, const uint64_t* tot, const MsmSortMax& mx, const MsmScalarBufs& bufs) {
     hipStream_t st = ctx->stream;
     const uint64_t ntiles = tot[SP_SCANTILE];
     {
         TimedLaunch tl(ctx, "msm_digits");
-        hipLaunchKernelGGL(k_msm_digits, dim3(grid_for(tot[SP_DIGIT], 256, 1u << 16)), dim3(256), 0, st, b, bufs.digits);
+        hipLaunchKernelGGL(k_msm_digits, dim3((unsigned)tot[SP_TILE]), dim3(mx.tile < 1024 ? 256 : 1024), 4 * mx.groups, st, b,
+                           bufs.digits, bufs.count);
     }
-    {
-        TimedLaunch tl(ctx, "msm_hist");
-        hipLaunchKernelGGL(k_msm_hist, dim3((unsigned)tot[SP_TILEWG]), dim3(1024), max_nb * 4, st, b, (const uint32_t*)bufs.digits,
-                           bufs.hist);
-    }
-    {
+    if (ntiles) {
         TimedLaunch tl(ctx, "msm_scan");
-        hipLaunchKernelGGL(k_msm_colscan, dim3(grid_for(tot[SP_KEY], 256, 1u << 30)), dim3(256), 0, st, b, bufs.hist, bufs.count);
-        hipLaunchKernelGGL(k_scan_tiles, dim3((unsigned)ntiles), dim3(SCAN_THREADS), 0, st, b, (const uint32_t*)bufs.count,
-                           bufs.tiles, bufs.tiles + ntiles);
-        hipLaunchKernelGGL(k_scan_top, dim3(b.ninst), dim3(1024), 0, st, b, bufs.tiles, (const uint64_t*)(bufs.tiles + ntiles));
-        hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)ntiles), dim3(SCAN_THREADS), 0, st, b, (const uint32_t*)bufs.count,
-                           (const uint64_t*)bufs.tiles, bufs.offs);
+        hipLaunchKernelGGL(k_scan_tiles, dim3((unsigned)ntiles), dim3(SCAN_THREADS), 0, st, b, (const uint32_t*)bufs.count, bufs.tiles);
+        hipLaunchKernelGGL(k_scan_top, dim3(b.ninst), dim3(1024), 0, st, b, bufs.tiles);
+        hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)ntiles), dim3(SCAN_THREADS), 0, st, b, bufs.count, (const uint64_t*)bufs.tiles);
+        hipLaunchKernelGGL(k_msm_pieces, dim3(b.ninst), dim3(1024), 0, st, b, (const uint32_t*)bufs.count, bufs.sub, bufs.offs);
     }
-    {
-        TimedLaunch tl(ctx, "msm_scatter");
-        hipLaunchKernelGGL(k_msm_scatter, dim3((unsigned)tot[SP_TILEWG]), dim3(1024), max_nb * 4, st, b,
-                           (const uint32_t*)bufs.digits, (const uint32_t*)bufs.hist, (const uint32_t*)bufs.offs, bufs.sorted);
-        if (bufs.coarse) {
-            hipLaunchKernelGGL(k_msm_scatter_coarse, dim3((unsigned)tot[SP_TILEWG]), dim3(SC_THREADS), 0, st, b,
-                               (const uint32_t*)bufs.digits, (const uint32_t*)bufs.hist, (const uint32_t*)bufs.offs, bufs.coarse);
-            hipLaunchKernelGGL(k_msm_scatter_fine, dim3((unsigned)tot[SP_CGROUP]), dim3(SC_THREADS), 0, st, b,
-                               (const uint2*)bufs.coarse, (const uint32_t*)bufs.offs, bufs.sorted);
-        }
+    TimedLaunch tl(ctx, "msm_scatter");
+    if (ntiles) {
+        hipLaunchKernelGGL(k_msm_scatter_coarse, dim3((unsigned)tot[SP_TILEWG]), dim3(SC_THREADS), 0, st, b, (const uint32_t*)bufs.digits,
+                           (const uint32_t*)bufs.count, bufs.cidx, bufs.ckey);
+        hipLaunchKernelGGL(k_msm_fine_count, dim3((unsigned)tot[SP_SUB]), dim3(512), 4 * mx.fine, st, b, (const uint32_t*)bufs.count,
+                           (const uint32_t*)bufs.sub, (const uint32_t*)bufs.cidx, (const uint16_t*)bufs.ckey, bufs.rows);
+        hipLaunchKernelGGL(k_msm_fine_offsets, dim3((unsigned)tot[SP_GROUP]), dim3(256), 8 * mx.fine, st, b, (const uint32_t*)bufs.count,
+                           (const uint32_t*)bufs.sub, bufs.rows, bufs.offs);
+        hipLaunchKernelGGL(k_msm_scatter_fine, dim3((unsigned)tot[SP_SUB]), dim3(SC_THREADS), 12 * mx.fine, st, b,
+                           (const uint32_t*)bufs.count, (const uint32_t*)bufs.sub, (const uint32_t*)bufs.rows, (const uint32_t*)bufs.cidx,
+                           (const uint16_t*)bufs.ckey, bufs.sorted);
     }
+    if (tot[SP_SMALL])
+        hipLaunchKernelGGL(k_msm_sort_small, dim3((unsigned)tot[SP_SMALL]), dim3(1024), 8 * mx.small_nb, st, b,
+                           (const uint32_t*)bufs.digits, (const uint32_t*)bufs.count, bufs.offs, bufs.sorted);
 }
 
 // Built-in plan (autotuned entries override it per size class).
 // c minimises n*W (bucket entries, one mixed addition each) + 3*W*2^(c-1)
 // (bucket reduction: two full additions per bucket plus its share of the run
-// weights), within the LDS histogram limit. K makes the accumulation about
+// weights). K makes the accumulation about
 // 2^18..2^19 lanes (4 waves per SIMD on every CU), each adding exactly K
 // entries.
-MsmPlan msm_plan(size_t n, int force_c, int force_g, size_t lds_bytes) {
+MsmPlan msm_plan(size_t n, int force_c, int force_g) {
     MsmPlan p;
-    int cmax = MSM_MAX_C;
-    while (cmax > MSM_MIN_C && ((size_t)4 << (cmax - 1)) > lds_bytes) --cmax;   // histogram must fit in LDS
+    const int cmax = MSM_MAX_C;
     int c = MSM_MIN_C;
     double best = -1;
     for (int cc = MSM_MIN_C; cc <= cmax; ++cc) {
@@ -533,13 +631,6 @@ MsmPlan msm_plan(size_t n, int force_c, int force_g, size_t lds_bytes) {
     if (force_g) g = force_g;
     if (g > p.NB) g = p.NB;   // a run never spans more buckets than a window has
     p.g = g;
-    // scalar tiles per window for the LDS histogram / scatter workgroups
-    // (about 512 workgroups per MSM; every tile at least 4096 scalars and 4x
-    // the bucket count, so the per-tile histograms stay smaller than the digits)
-    uint32_t T = (512 + p.W - 1) / p.W;
-    while (T > 1 && (n / T < 4096 || n / T < 4 * (size_t)p.NB)) T >>= 1;
-    p.T = T;
-    p.tile = (uint32_t)((n + T - 1) / T);
     return p;
 }
 
@@ -555,19 +646,19 @@ static int size_class(size_t n) {
     return cls < 32 ? cls : 31;
 }
 
-static bool plan_from_entry(const hzk_tune_entry& t, size_t n, int force_g, size_t lds_bytes, MsmPlan* out) {
-    if (!t.c || ((size_t)4 << (t.c - 1)) > lds_bytes) return false;
-    MsmPlan q = msm_plan(n, t.c, t.g ? (int)t.g : force_g, lds_bytes);
+static bool plan_from_entry(const hzk_tune_entry& t, size_t n, int force_g, MsmPlan* out) {
+    if (!t.c) return false;
+    MsmPlan q = msm_plan(n, t.c, t.g ? (int)t.g : force_g);
     if (t.K) q.K = t.K;
     *out = q;
     return true;
 }
 
-MsmPlan msm_plan_builtin(int g2, size_t n, int regime, size_t lds_bytes) {
-    MsmPlan p = msm_plan(n, 0, 0, lds_bytes);
+MsmPlan msm_plan_builtin(int g2, size_t n, int regime) {
+    MsmPlan p = msm_plan(n, 0, 0);
     const int cls = size_class(n);
-    if (regime == MSM_REGIME_BATCH && plan_from_entry(BUILTIN_PLANS[1][g2 ? 1 : 0][cls], n, 0, lds_bytes, &p)) return p;
-    plan_from_entry(BUILTIN_PLANS[0][g2 ? 1 : 0][cls], n, 0, lds_bytes, &p);
+    if (regime == MSM_REGIME_BATCH && plan_from_entry(BUILTIN_PLANS[1][g2 ? 1 : 0][cls], n, 0, &p)) return p;
+    plan_from_entry(BUILTIN_PLANS[0][g2 ? 1 : 0][cls], n, 0, &p);
     return p;
 }
 
@@ -577,13 +668,13 @@ MsmPlan msm_plan_builtin(int g2, size_t n, int regime, size_t lds_bytes) {
 // heuristic. A caller-forced window size (or hzk_set_tuning) bypasses the
 // tables.
 MsmPlan msm_plan_ctx(hzk_ctx* ctx, int g2, size_t n, int force_c, int regime) {
-    MsmPlan p = msm_plan(n, force_c ? force_c : ctx->force_window, ctx->force_seg, ctx->lds_per_block);
+    MsmPlan p = msm_plan(n, force_c ? force_c : ctx->force_window, ctx->force_seg);
     if (!force_c && !ctx->force_window) {
         const int cls = size_class(n), gi = g2 ? 1 : 0;
         for (int r = regime; r >= MSM_REGIME_SINGLE; --r) {
             hzk_tune_entry t = ctx->tune[r][gi][cls];
             if (!t.c && !ctx->force_seg) t = BUILTIN_PLANS[r][gi][cls];
-            if (plan_from_entry(t, n, ctx->force_seg, ctx->lds_per_block, &p)) break;
+            if (plan_from_entry(t, n, ctx->force_seg, &p)) break;
         }
     }
     return p;

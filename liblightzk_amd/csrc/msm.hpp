@@ -10,7 +10,8 @@ struct hzk_ctx;
 namespace hzk {
 
 constexpr int MSM_MIN_C = 4;
-constexpr int MSM_MAX_C = 16;   // 2^(c-1) LDS counters per histogram workgroup
+constexpr int MSM_MAX_C = 16;         // a caller's window sizes and the autotuner's
+constexpr int MSM_PLAN_MAX_C = 20;    // built-in plans
 
 struct MsmPlan {
     int c;          // window bits
@@ -18,12 +19,10 @@ struct MsmPlan {
     uint32_t NB;    // buckets per window, 2^(c-1)
     uint32_t K;     // sorted entries per accumulation lane (chunk length)
     uint32_t g;     // buckets per bucket-reduction run
-    uint32_t T;     // scalar tiles per window (histogram / scatter workgroups)
-    uint32_t tile;  // scalars per tile
 };
 // Plan for n points: autotuned entry for the size class if one is loaded,
 // else the built-in heuristic; force_c / force_g override (0 = automatic).
-MsmPlan msm_plan(size_t n, int force_c, int force_g, size_t lds_bytes);
+MsmPlan msm_plan(size_t n, int force_c, int force_g);
 // plan regimes: an MSM with the GPU to itself, or an instance of a wide
 // batch: two or more instances whose digits total at least
 // MSM_WIDE_BATCH_ENTRIES, or many instances (MSM_WIDE_BATCH_COUNT, G1 / G2)
@@ -41,21 +40,24 @@ inline bool msm_wide_batch(int g2, size_t count, uint64_t entries) {
 }
 MsmPlan msm_plan_ctx(hzk_ctx* ctx, int g2, size_t n, int force_c, int regime = MSM_REGIME_SINGLE);
 // the built-in plan of a regime (no context overrides)
-MsmPlan msm_plan_builtin(int g2, size_t n, int regime, size_t lds_bytes);
+MsmPlan msm_plan_builtin(int g2, size_t n, int regime);
 
 // Work spaces of the batched stages; each instance owns a contiguous range
 // [begin[s][i], begin[s][i+1]) of every space.
 enum MsmSpace {
-    SP_DIGIT = 0,   // one lane per scalar
-    SP_TILEWG,      // one workgroup per (tile, window)
-    SP_KEY,         // nk + 1 entries per instance (counts, offsets, bucket sums)
-    SP_SCANTILE,    // scan tiles over the key space
+    SP_TILE = 0,    // one workgroup per tile of scalars (recode)
+    SP_TILEWG,      // one workgroup per (tile, window) (coarse scatter)
+    SP_CNT,         // W * CG * T + 1 coarse counts, then starts
+    SP_SCANTILE,    // scan tiles over them
+    SP_GROUP,       // W * CG + 1 coarse groups
+    SP_SUB,         // pieces of MSM_SUB entries of a group (upper bound)
+    SP_ROW,         // FB counters per piece
+    SP_SMALL,       // one workgroup per window of a small instance
+    SP_KEY,         // nk + 1 entries per instance (offsets, bucket sums)
     SP_CHUNK,       // accumulation chunks of K sorted entries (upper bound)
     SP_BRED,        // window values (device-side combine)
     SP_WIN,         // window-sum partials (S per window)
     SP_ENTRY,       // n * W digit / sorted-entry slots
-    SP_HIST,        // T * nk per-tile histogram counters
-    SP_CGROUP,      // W * 256 coarse key groups (two-pass scatter)
     SP_COUNT
 };
 
@@ -70,8 +72,10 @@ struct MsmInst {
     // pipeline) serves Lg consecutive digit windows, so W = ceil(Wd / Lg) and
     // n = nd * Lg virtual points. Plain bases: nd = n, Wd = W, Lg = 1.
     uint32_t nd, Wd, Lg;
-    uint32_t tp;           // scatter in two passes (coarse groups, then buckets): 0 no, 1 yes
-                           // (8-byte coarse entries), 2 yes (packed 4-byte coarse entries)
+    uint32_t CG, FB;       // coarse groups per window, buckets per group (powers of two, CG * FB = NB)
+    uint32_t small;        // 1: sorted by one workgroup per window (CG = 1)
+    uint32_t ctile;        // tiles per coarse-scatter workgroup
+    uint32_t ib;           // bits of a point index where it shares a coarse entry's word with the bucket, else 0
     // Digit window j covers bits [j*wb + min(j, wx), +wb + (j < wx)): the 255
     // bits of a signed recoding of a scalar < 2^254 split as evenly as the W
     // windows allow (widths c and c - 1), so the top window is not a sliver
@@ -88,32 +92,54 @@ struct MsmBatchDev {
     uint32_t* stats;          // per instance {entries, chunks, largest bucket, 0}
 };
 
-// Launch the scalar-side stages (digits, LDS histograms, scans, scatter) for a
-// whole batch. Buffers are indexed through the work spaces above.
+// Limits of the two-level sort. Coarse groups: 256 keep the runs that a round
+// of the coarse scatter writes at 128 bytes (512 only where that lets an entry
+// fit one word); FB counters of a group times three and a round of the fine
+// scatter share the LDS. A piece is two rounds.
+constexpr uint32_t MSM_MAX_COARSE = 512, MSM_MAX_FINE = 2048;
+constexpr uint32_t MSM_MAX_GROUPS = 8192;   // W * CG counters of the recode
+constexpr uint32_t MSM_SUB = 16384;
+static_assert((1u << (MSM_PLAN_MAX_C - 1)) <= MSM_MAX_COARSE * MSM_MAX_FINE, "a window's buckets fit the two levels");
+// Small instances: the six launches of the two levels cost more than one
+// workgroup per window (measured: MEASURED_SMALL)
+constexpr uint32_t MSM_SMALL_N = 1u << 15, MSM_SMALL_NB = 1u << 13;
+inline uint32_t msm_log2_ceil(uint64_t n) {
+    uint32_t k = 0;
+    while (((uint64_t)1 << k) < n) ++k;
+    return k;
+}
+// point index, bucket of the group and sign in one 32-bit word
+inline bool msm_packs(uint64_t n, uint32_t FB) { return msm_log2_ceil(n) + msm_log2_ceil(FB) <= 31; }
+// coarse groups per window: about 4096 entries each, within the limits
+inline uint32_t msm_coarse_groups(uint64_t n, uint32_t NB, uint32_t W) {
+    uint32_t cg = 1;
+    while (cg < 256 && cg < NB && n / cg > 4096 && W * cg * 2 <= MSM_MAX_GROUPS) cg *= 2;
+    while (NB / cg > MSM_MAX_FINE) cg *= 2;
+    while (cg < MSM_MAX_COARSE && cg < NB && !msm_packs(n, NB / cg) && W * cg * 2 <= MSM_MAX_GROUPS) cg *= 2;
+    return cg;
+}
+// tiles of scalars: about 256 each, at most 512 of them (their counts are scanned)
+inline uint32_t msm_tiles(uint64_t nd) {
+    const uint64_t t = (nd + 255) / 256;
+    return (uint32_t)(t < 512 ? t : 512);
+}
+
+// Launch the scalar-side stages (recode, scans, scatters) for a whole batch.
+// Buffers are indexed through the work spaces above.
 struct MsmScalarBufs {
     uint32_t* digits;    // SP_ENTRY
-    uint32_t* hist;      // SP_HIST
-    uint32_t* count;     // SP_KEY
+    uint32_t* count;     // SP_CNT
+    uint64_t* tiles;     // SP_SCANTILE
+    uint32_t* sub;       // SP_GROUP
+    uint32_t* rows;      // SP_ROW
+    uint32_t* cidx;      // SP_ENTRY coarse entries: point index and sign
+    uint16_t* ckey;      // SP_ENTRY: bucket within the group
     uint32_t* offs;      // SP_KEY
-    uint64_t* tiles;     // 2 * SP_SCANTILE
     uint32_t* sorted;    // SP_ENTRY
-    uint2* coarse;       // SP_ENTRY 8-byte entries, or null when no instance uses the two-pass scatter
 };
-constexpr uint32_t MSM_COARSE = 256;   // coarse key groups per window
-// Instances with many buckets per window and enough points that each coarse
-// group holds a few thousand entries scatter in two passes; below that the
-// per-group fixed cost outweighs the write coalescing.
-// Two-pass scatter: alone, an instance pays for the extra pass from 2^19
-// points on; in a batch whose instances scatter together (batch_entries
-// digits in all), their random 4-byte writes share the L2 and the coalesced
-// two-pass form wins from MSM_TP_BATCH_MIN_N points on.
-constexpr uint64_t MSM_TP_BATCH_ENTRIES = (uint64_t)1 << 23;
-constexpr uint32_t MSM_TP_BATCH_MIN_N = 1u << 15;
-inline bool msm_two_pass(uint32_t n, uint32_t NB, uint64_t batch_entries) {
-    if (NB < 2048) return false;
-    return n >= (1u << 19) || (batch_entries >= MSM_TP_BATCH_ENTRIES && n >= MSM_TP_BATCH_MIN_N);
-}
-void msm_launch_scalar_stages(hzk_ctx* ctx, const MsmBatchDev& b, const uint64_t* host_totals, uint32_t max_nb,
+// largest of the batch, for the launches' LDS
+struct MsmSortMax { uint32_t groups = 1, fine = 1, small_nb = 1, tile = 1; };
+void msm_launch_scalar_stages(hzk_ctx* ctx, const MsmBatchDev& b, const uint64_t* host_totals, const MsmSortMax& mx,
                               const MsmScalarBufs& bufs);
 constexpr uint32_t MSM_SCAN_TILE = 1024;
 // one-time kernel attribute setup (call outside graph capture)

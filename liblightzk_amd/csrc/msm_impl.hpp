@@ -620,13 +620,14 @@ struct MsmBatchLayout {
     std::vector<MsmInst> inst;
     std::vector<uint64_t> begin;   // [SP_COUNT][ninst + 1]
     uint64_t tot[SP_COUNT];
-    uint32_t max_nb = 1;
+    MsmSortMax sort_max;
     uint32_t hot_levels = 0;       // levels of k_msm_hot_sum (upper bound)
-    bool two_pass = false;         // some instance scatters in two passes
+    bool two_level = false;        // some instance is sorted in two levels
+    bool unpacked = false;         // some coarse entries take two arrays
     int regime = 0;                // plan regime (MSM_REGIME_*)
     size_t bytes = 0;              // scratch needed
     // scratch offsets
-    size_t o_inst, o_begin, o_stats, o_digits, o_hist, o_count, o_offs, o_tiles, o_sorted, o_coarse, o_chunk2key, o_bucket,
+    size_t o_inst, o_begin, o_stats, o_digits, o_count, o_tiles, o_sub, o_rows, o_cidx, o_ckey, o_offs, o_sorted, o_chunk2key, o_bucket,
         o_carry, o_tsum, o_win;
     // base arrays converted for the accumulation, one per distinct source
     // array (its largest referenced point count), and which one each instance reads
@@ -669,8 +670,6 @@ static MsmBatchLayout msm_layout(hzk_ctx* ctx, const MsmJob* jobs, size_t count)
         d.K = p.K;
         d.g = p.g;
         d.G = p.NB / p.g;
-        d.T = p.T;
-        d.tile = p.tile;
         d.nd = d.n;
         d.Wd = d.W;
         d.Lg = 1;
@@ -689,49 +688,46 @@ static MsmBatchLayout msm_layout(hzk_ctx* ctx, const MsmJob* jobs, size_t count)
             uint32_t K = 4;
             while (K < 4096 && entries / (2 * (uint64_t)K) >= ((uint64_t)1 << 18)) K <<= 1;
             d.K = K;
-            uint32_t T = (512 + d.W - 1) / d.W;
-            while (T > 1 && (d.n / T < 4096 || d.n / T < 4 * d.NB)) T >>= 1;
-            d.T = T;
-            d.tile = (d.n + T - 1) / T;
         }
         // parts per window: one run of g buckets per slot of a window-sum
         // workgroup, at most 64 parts (host combine, lanes of the device combine)
         const uint32_t slots = regime == MSM_REGIME_BATCH ? LdsLanes<F, 64>::SLOTS : LdsLanes<F, 256>::SLOTS;
         d.S = 1;
         while (d.S < 64 && d.G / d.S > slots) d.S *= 2;
+        d.T = msm_tiles(d.nd);
+        d.tile = (d.nd + d.T - 1) / d.T;
+        d.small = d.n <= MSM_SMALL_N && d.NB <= MSM_SMALL_NB;
+        d.CG = d.small ? 1 : msm_coarse_groups(d.n, d.NB, d.W);
+        d.FB = d.NB / d.CG;
+        // at least a round of the coarse scatter per workgroup, and about 2048 workgroups
+        d.ctile = std::max({1u, 8192 / d.tile, d.T * d.W / 2048});
+        d.ib = msm_packs(d.n, d.FB) ? std::max(1u, msm_log2_ceil(d.n)) : 0;
+        L.sort_max.tile = std::max(L.sort_max.tile, d.tile);
+        L.sort_max.groups = std::max(L.sort_max.groups, d.W * d.CG);
+        if (d.small) L.sort_max.small_nb = std::max(L.sort_max.small_nb, d.NB);
+        else L.sort_max.fine = std::max(L.sort_max.fine, d.FB), L.two_level = true, L.unpacked |= !d.ib;
         uint64_t entries = (uint64_t)d.n * d.W;
+        const uint64_t groups = (uint64_t)d.W * d.CG;
         uint64_t sz[SP_COUNT];
-        sz[SP_DIGIT] = d.nd;
-        sz[SP_TILEWG] = (uint64_t)d.T * d.W;
+        sz[SP_TILE] = d.T;
+        sz[SP_TILEWG] = d.small ? 0 : (uint64_t)((d.T + d.ctile - 1) / d.ctile) * d.W;
+        sz[SP_CNT] = groups * d.T + 1;
+        sz[SP_SCANTILE] = d.small ? 0 : (groups * d.T + MSM_SCAN_TILE) / MSM_SCAN_TILE;
+        sz[SP_GROUP] = d.small ? 0 : groups + 1;
+        sz[SP_SUB] = d.small ? 0 : entries / MSM_SUB + groups;
+        sz[SP_ROW] = sz[SP_SUB] * d.FB;
+        sz[SP_SMALL] = d.small ? d.W : 0;
         sz[SP_KEY] = (uint64_t)d.nk + 1;
-        sz[SP_SCANTILE] = ((uint64_t)d.nk + MSM_SCAN_TILE) / MSM_SCAN_TILE;
         sz[SP_CHUNK] = (entries + d.K - 1) / d.K;
         sz[SP_BRED] = (uint64_t)d.W;
         sz[SP_WIN] = (uint64_t)d.W * d.S;
         sz[SP_ENTRY] = (entries + 63) & ~(uint64_t)63;   // 256-B aligned per instance (vector index loads)
-        sz[SP_HIST] = (uint64_t)d.T * d.nk;
-        d.tp = 0;   // two-pass flag and coarse groups: set below, once the batch's digit total is known
-        sz[SP_CGROUP] = 0;
         for (int s = 0; s < SP_COUNT; ++s) L.begin[(size_t)s * (count + 1) + i + 1] = L.begin[(size_t)s * (count + 1) + i] + sz[s];
-        if (d.NB > L.max_nb) L.max_nb = d.NB;
         uint64_t maxspan = (d.n + d.K - 1) / d.K + 1;   // a bucket holds at most n entries
         uint32_t lv = 0;
         if (maxspan > HOT)
             for (uint64_t stride = 1; stride < maxspan; stride *= hot_seg<F>()) ++lv;
         if (lv > L.hot_levels) L.hot_levels = lv;
-    }
-    // two-pass scatter per instance, then the coarse-group space it needs
-    uint64_t batch_entries = 0;
-    for (const MsmInst& d : L.inst) batch_entries += (uint64_t)d.n * d.W;
-    for (size_t i = 0; i < count; ++i) {
-        MsmInst& d = L.inst[i];
-        d.tp = msm_two_pass(d.n, d.NB, batch_entries) ? 1u : 0u;
-        // coarse entries fit one word (index | fine key << 24 | sign << 31)
-        // when point indices stay below 2^24 and a group has at most 128 buckets
-        if (d.tp && d.n <= (1u << 24) && d.NB / MSM_COARSE <= 128) d.tp = 2;
-        if (d.tp) L.two_pass = true;
-        const size_t s = SP_CGROUP;
-        L.begin[s * (count + 1) + i + 1] = L.begin[s * (count + 1) + i] + (d.tp ? (uint64_t)d.W * MSM_COARSE : 0);
     }
     for (int s = 0; s < SP_COUNT; ++s) L.tot[s] = L.begin[(size_t)s * (count + 1) + count];
     size_t off = 0;
@@ -740,12 +736,14 @@ static MsmBatchLayout msm_layout(hzk_ctx* ctx, const MsmJob* jobs, size_t count)
     L.o_begin = take(L.begin.size() * 8);
     L.o_stats = take(count * 16);
     L.o_digits = take(L.tot[SP_ENTRY] * 4);
-    L.o_hist = take(L.tot[SP_HIST] * 4);
-    L.o_count = take(L.tot[SP_KEY] * 4);
+    L.o_count = take(L.tot[SP_CNT] * 4);
+    L.o_tiles = take(L.tot[SP_SCANTILE] * 8);
+    L.o_sub = take(L.tot[SP_GROUP] * 4);
+    L.o_rows = take(L.tot[SP_ROW] * 4);
+    L.o_cidx = take(L.two_level ? L.tot[SP_ENTRY] * 4 : 0);
+    L.o_ckey = take(L.unpacked ? L.tot[SP_ENTRY] * 2 : 0);
     L.o_offs = take(L.tot[SP_KEY] * 4);
-    L.o_tiles = take(2 * L.tot[SP_SCANTILE] * 8);
     L.o_sorted = take(L.tot[SP_ENTRY] * 4);
-    L.o_coarse = take(L.two_pass ? L.tot[SP_ENTRY] * 8 : 0);
     const size_t raw = (size_t)raw_vec<F>() * 16;   // bytes per raw accumulator state
     L.o_chunk2key = take(L.tot[SP_CHUNK] * 4);
     L.o_bucket = take(L.tot[SP_KEY] * raw);
@@ -785,12 +783,14 @@ static void msm_device_stages(hzk_ctx* ctx, const MsmBatchLayout& L, char* base)
     b.stats = (uint32_t*)(base + L.o_stats);
     MsmScalarBufs sb;
     sb.digits = (uint32_t*)(base + L.o_digits);
-    sb.hist = (uint32_t*)(base + L.o_hist);
     sb.count = (uint32_t*)(base + L.o_count);
-    sb.offs = (uint32_t*)(base + L.o_offs);
     sb.tiles = (uint64_t*)(base + L.o_tiles);
+    sb.sub = (uint32_t*)(base + L.o_sub);
+    sb.rows = (uint32_t*)(base + L.o_rows);
+    sb.cidx = (uint32_t*)(base + L.o_cidx);
+    sb.ckey = (uint16_t*)(base + L.o_ckey);
+    sb.offs = (uint32_t*)(base + L.o_offs);
     sb.sorted = (uint32_t*)(base + L.o_sorted);
-    sb.coarse = L.two_pass ? (uint2*)(base + L.o_coarse) : nullptr;
     uint32_t* chunk2key = (uint32_t*)(base + L.o_chunk2key);
     uint4* bucket = (uint4*)(base + L.o_bucket);
     uint4* carry = (uint4*)(base + L.o_carry);
@@ -807,7 +807,7 @@ static void msm_device_stages(hzk_ctx* ctx, const MsmBatchLayout& L, char* base)
         else
             hipLaunchKernelGGL(k_msm_convert_g2, grid, dim3(256), 0, st, tasks, (uint32_t)L.conv.size(), L.conv_total);
     }
-    msm_launch_scalar_stages(ctx, b, L.tot, L.max_nb, sb);
+    msm_launch_scalar_stages(ctx, b, L.tot, L.sort_max, sb);
     {
         TimedLaunch tl(ctx, "msm_accumulate");
         uint64_t blocks = (L.tot[SP_CHUNK] + 255) / 256;
@@ -895,9 +895,6 @@ int msm_batch_run(hzk_ctx* ctx, const MsmJob* jobs, size_t count, int dests_on_h
     for (size_t i = 0; i < count; ++i)   // bucket offsets are 32-bit
         HZK_CHECK(ctx, (uint64_t)L.inst[i].n * L.inst[i].W <= 0xffff0000ull, HZK_ERR_UNSUPPORTED,
                   "msm: n=%u with %u windows exceeds 2^32 bucket entries", L.inst[i].n, L.inst[i].W);
-    HZK_CHECK(ctx, (size_t)L.max_nb * 4 <= ctx->lds_per_block, HZK_ERR_UNSUPPORTED,
-              "msm: a %u-bucket window needs %u B of LDS per workgroup, device allows %zu", L.max_nb, L.max_nb * 4,
-              ctx->lds_per_block);
     int rc = 0;
     if (ext_scratch) {
         HZK_CHECK(ctx, L.bytes <= ext_bytes && !capture, HZK_ERR_UNSUPPORTED,

@@ -119,8 +119,7 @@ int autotune(hzk_ctx* ctx, int regime, int group, int log_min, int log_max, doub
     const int saved_w = ctx->force_window, saved_s = ctx->force_seg, saved_r = ctx->force_regime;
     ctx->force_window = ctx->force_seg = 0;
     ctx->force_regime = regime;
-    int cmax = MSM_MAX_C;
-    while (cmax > MSM_MIN_C && ((size_t)4 << (cmax - 1)) > ctx->lds_per_block) --cmax;
+    const int cmax = MSM_MAX_C;
 
     for (int L = log_min; L <= log_max && !rc; ++L) {
         const size_t n = (size_t)1 << L;
@@ -147,7 +146,7 @@ int autotune(hzk_ctx* ctx, int regime, int group, int log_min, int log_max, doub
         //    K and g in the batch regime, where lanes are plentiful)
         for (int c = base.c - 3; c <= base.c + 2; ++c) {
             if (c < MSM_MIN_C || c > cmax || c == base.c) continue;
-            MsmPlan q = msm_plan(n, c, 0, ctx->lds_per_block);
+            MsmPlan q = msm_plan(n, c, 0);
             if (regime == MSM_REGIME_BATCH) try_entry({c, base.K, std::min<uint32_t>(base.g, 1u << (c - 1))});
             else try_entry({c, q.K, q.g});
         }
