@@ -528,10 +528,18 @@ __global__ void __launch_bounds__(1024) k_msm_sort_small(MsmBatchDev b, const ui
     if (s0) atomicAdd(&before, s0);
     const uint64_t ebase = space(b, SP_ENTRY)[ii];
     const uint32_t* dj = digits + ebase + (size_t)j * n;
-    for (uint32_t i = tid; i < n; i += 1024) {
-        const uint32_t m = dj[i] & ~DIGIT_NEG;
-        if (m) atomicAdd(&cnt[m - 1], 1u);
-    }
+    // the thread's nonzero digits, eight loads at a time
+    auto each = [&](auto f) {
+        for (uint32_t base = tid; base < n; base += 8 * 1024) {
+            uint32_t dg[8];
+#pragma unroll
+            for (uint32_t k = 0; k < 8; ++k) dg[k] = base + k * 1024 < n ? dj[base + k * 1024] : 0;
+#pragma unroll
+            for (uint32_t k = 0; k < 8; ++k)
+                if (dg[k]) f(base + k * 1024, dg[k]);
+        }
+    };
+    each([&](uint32_t, uint32_t dg) { atomicAdd(&cnt[(dg & ~DIGIT_NEG) - 1], 1u); });
     __syncthreads();
     lds_exclusive_scan<1024>(cnt, cur, part, d.NB);
     uint32_t* of = offs + space(b, SP_KEY)[ii] + (size_t)j * d.NB;
@@ -552,10 +560,7 @@ __global__ void __launch_bounds__(1024) k_msm_sort_small(MsmBatchDev b, const ui
         }
     }
     uint32_t* out = sorted + ebase;
-    for (uint32_t i = tid; i < n; i += 1024) {
-        const uint32_t dg = dj[i], m = dg & ~DIGIT_NEG;
-        if (m) out[atomicAdd(&cur[m - 1], 1u)] = i | (dg & DIGIT_NEG);
-    }
+    each([&](uint32_t i, uint32_t dg) { out[atomicAdd(&cur[(dg & ~DIGIT_NEG) - 1], 1u)] = i | (dg & DIGIT_NEG); });
 }
 
 // ------------------------------------------------------------------ host side

@@ -100,9 +100,10 @@ constexpr uint32_t MSM_MAX_COARSE = 512, MSM_MAX_FINE = 2048;
 constexpr uint32_t MSM_MAX_GROUPS = 8192;   // W * CG counters of the recode
 constexpr uint32_t MSM_SUB = 16384;
 static_assert((1u << (MSM_PLAN_MAX_C - 1)) <= MSM_MAX_COARSE * MSM_MAX_FINE, "a window's buckets fit the two levels");
-// Small instances: the six launches of the two levels cost more than one
-// workgroup per window (measured: MEASURED_SMALL)
-constexpr uint32_t MSM_SMALL_N = 1u << 15, MSM_SMALL_NB = 1u << 13;
+// Small instances take one workgroup per window instead of the two levels'
+// seven launches: up to 2^15 points, or 2^17 in a wide batch, whose windows
+// fill the GPU together
+constexpr uint32_t MSM_SMALL_N = 1u << 15, MSM_SMALL_BATCH_N = 1u << 17, MSM_SMALL_NB = 1u << 13;
 inline uint32_t msm_log2_ceil(uint64_t n) {
     uint32_t k = 0;
     while (((uint64_t)1 << k) < n) ++k;

@@ -696,7 +696,7 @@ static MsmBatchLayout msm_layout(hzk_ctx* ctx, const MsmJob* jobs, size_t count)
         while (d.S < 64 && d.G / d.S > slots) d.S *= 2;
         d.T = msm_tiles(d.nd);
         d.tile = (d.nd + d.T - 1) / d.T;
-        d.small = d.n <= MSM_SMALL_N && d.NB <= MSM_SMALL_NB;
+        d.small = d.n <= (regime == MSM_REGIME_BATCH ? MSM_SMALL_BATCH_N : MSM_SMALL_N) && d.NB <= MSM_SMALL_NB;
         d.CG = d.small ? 1 : msm_coarse_groups(d.n, d.NB, d.W);
         d.FB = d.NB / d.CG;
         // at least a round of the coarse scatter per workgroup, and about 2048 workgroups
