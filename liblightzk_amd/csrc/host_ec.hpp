@@ -38,41 +38,58 @@ struct Fp {
     bool operator==(const Fp& o) const { return std::memcmp(v, o.v, 32) == 0; }
     bool operator!=(const Fp& o) const { return !(*this == o); }
 
-    static bool geq_p(const uint64_t* t) {
-        for (int i = 3; i >= 0; --i) { if (t[i] != P.p[i]) return t[i] > P.p[i]; }
-        return true;
-    }
-    static void sub_p(uint64_t* t) {
-        uint64_t bw = 0;
-        for (int i = 0; i < 4; ++i) { u128 d = (u128)t[i] - P.p[i] - bw; t[i] = (uint64_t)d; bw = (uint64_t)(d >> 127); }
-    }
-    // Montgomery product, operand scanning with interleaved reduction
-    friend Fp operator*(const Fp& a, const Fp& b) {
-        uint64_t t[5] = {0, 0, 0, 0, 0};
-        for (int i = 0; i < 4; ++i) {
-            u128 c = 0;
-            for (int j = 0; j < 4; ++j) { c = (u128)a.v[j] * b.v[i] + t[j] + (uint64_t)(c >> 64); t[j] = (uint64_t)c; }
-            uint64_t top = (uint64_t)(c >> 64);
-            uint64_t m = t[0] * P.inv;
-            c = (u128)m * P.p[0] + t[0];
-            for (int j = 1; j < 4; ++j) { c = (u128)m * P.p[j] + t[j] + (uint64_t)(c >> 64); t[j - 1] = (uint64_t)c; }
-            c = (u128)t[4] + top + (uint64_t)(c >> 64);
-            t[3] = (uint64_t)c;
-            t[4] = (uint64_t)(c >> 64);
-        }
-        if (t[4] || geq_p(t)) sub_p(t);
-        Fp r; std::memcpy(r.v, t, 32); return r;
-    }
-    friend Fp operator+(const Fp& a, const Fp& b) {
-        Fp r; u128 c = 0;
-        for (int i = 0; i < 4; ++i) { c += (u128)a.v[i] + b.v[i]; r.v[i] = (uint64_t)c; c >>= 64; }
-        if (geq_p(r.v)) sub_p(r.v);
+    // t - p where t >= p, else t (t < 2p), without a branch: the comparison is
+    // a coin toss, and a mispredicted one costs as much as a product
+    static Fp reduced(uint64_t t0, uint64_t t1, uint64_t t2, uint64_t t3) {
+        uint64_t d[4], bw = 0;
+        const uint64_t t[4] = {t0, t1, t2, t3};
+        for (int i = 0; i < 4; ++i) { u128 x = (u128)t[i] - P.p[i] - bw; d[i] = (uint64_t)x; bw = (uint64_t)(x >> 64) & 1; }
+        const uint64_t keep = 0 - bw;   // all ones: t < p
+        Fp r;
+        for (int i = 0; i < 4; ++i) r.v[i] = (t[i] & keep) | (d[i] & ~keep);
         return r;
     }
+    // Montgomery product, operand scanning with interleaved reduction; both
+    // carry words stay below 2^64 because the top word of p is below 2^62
+    friend Fp operator*(const Fp& a, const Fp& b) {
+        uint64_t t0 = 0, t1 = 0, t2 = 0, t3 = 0;
+#pragma GCC unroll 4
+        for (int i = 0; i < 4; ++i) {
+            const uint64_t y = b.v[i];
+            u128 x = (u128)a.v[0] * y + t0;
+            const uint64_t lo = (uint64_t)x, m = lo * P.inv;
+            uint64_t ca = (uint64_t)(x >> 64);
+            u128 z = (u128)m * P.p[0] + lo;
+            uint64_t cm = (uint64_t)(z >> 64);
+            x = (u128)a.v[1] * y + t1 + ca;
+            ca = (uint64_t)(x >> 64);
+            z = (u128)m * P.p[1] + (uint64_t)x + cm;
+            t0 = (uint64_t)z, cm = (uint64_t)(z >> 64);
+            x = (u128)a.v[2] * y + t2 + ca;
+            ca = (uint64_t)(x >> 64);
+            z = (u128)m * P.p[2] + (uint64_t)x + cm;
+            t1 = (uint64_t)z, cm = (uint64_t)(z >> 64);
+            x = (u128)a.v[3] * y + t3 + ca;
+            ca = (uint64_t)(x >> 64);
+            z = (u128)m * P.p[3] + (uint64_t)x + cm;
+            t2 = (uint64_t)z;
+            t3 = (uint64_t)(z >> 64) + ca;
+        }
+        return reduced(t0, t1, t2, t3);
+    }
+    friend Fp operator+(const Fp& a, const Fp& b) {
+        uint64_t t[4];
+        u128 c = 0;
+        for (int i = 0; i < 4; ++i) { c += (u128)a.v[i] + b.v[i]; t[i] = (uint64_t)c; c >>= 64; }
+        return reduced(t[0], t[1], t[2], t[3]);   // a + b < 2p < 2^255
+    }
     friend Fp operator-(const Fp& a, const Fp& b) {
-        Fp r; uint64_t bw = 0;
-        for (int i = 0; i < 4; ++i) { u128 d = (u128)a.v[i] - b.v[i] - bw; r.v[i] = (uint64_t)d; bw = (uint64_t)(d >> 127); }
-        if (bw) { u128 c = 0; for (int i = 0; i < 4; ++i) { c += (u128)r.v[i] + P.p[i]; r.v[i] = (uint64_t)c; c >>= 64; } }
+        uint64_t t[4], bw = 0;
+        for (int i = 0; i < 4; ++i) { u128 d = (u128)a.v[i] - b.v[i] - bw; t[i] = (uint64_t)d; bw = (uint64_t)(d >> 64) & 1; }
+        const uint64_t add = 0 - bw;
+        u128 c = 0;
+        Fp r;
+        for (int i = 0; i < 4; ++i) { c += (u128)t[i] + (P.p[i] & add); r.v[i] = (uint64_t)c; c >>= 64; }
         return r;
     }
     Fp neg() const { return zero() - *this; }
@@ -83,10 +100,93 @@ struct Fp {
         for (int i = 255; i >= 0; --i) { acc = acc.sqr(); if ((e[i / 64] >> (i % 64)) & 1) acc = acc * *this; }
         return acc;
     }
-    Fp inverse() const {   // a^(p-2); 0 -> 0
-        uint64_t e[4] = {P.p[0] - 2, P.p[1], P.p[2], P.p[3]};
-        return pow(e);
+    // 1/a; 0 -> 0. T. Pornin, "Optimized Binary GCD for Modular Inversion"
+    // (2020): 17 rounds of 31 halvings (2 * 254 - 1 are enough) on 64-bit
+    // stand-ins for a and b, their low 31 and leading 33 bits, after which the
+    // recorded factors update a, b exactly and u, v modulo p. 2.5 us against
+    // 13 us for a^(p-2).
+    Fp inverse() const {
+        uint64_t a[4], b[4];
+        std::memcpy(a, v, 32);
+        std::memcpy(b, P.p, 32);
+        Fp u{{1, 0, 0, 0}}, w = zero();
+        for (int round = 0; round < 17; ++round) {
+            uint64_t x, y;
+            {
+                int k = 3;
+                while (k > 0 && !(a[k] | b[k])) --k;
+                if (k == 0) x = a[0], y = b[0];
+                else {
+                    const int sh = __builtin_clzll(a[k] | b[k]);
+                    const uint64_t ha = sh ? (a[k] << sh) | (a[k - 1] >> (64 - sh)) : a[k];
+                    const uint64_t hb = sh ? (b[k] << sh) | (b[k - 1] >> (64 - sh)) : b[k];
+                    const uint64_t low = 0x7fffffffu;
+                    x = (a[0] & low) | (ha & ~low);
+                    y = (b[0] & low) | (hb & ~low);
+                }
+            }
+            int64_t f0 = 1, g0 = 0, f1 = 0, g1 = 1;
+            for (int i = 0; i < 31; ++i) {
+                const uint64_t odd = 0 - (x & 1), swap = odd & (0 - (uint64_t)(x < y));
+                const uint64_t tx = (x ^ y) & swap;
+                x ^= tx, y ^= tx;
+                const int64_t tf = (f0 ^ f1) & (int64_t)swap, tg = (g0 ^ g1) & (int64_t)swap;
+                f0 ^= tf, f1 ^= tf, g0 ^= tg, g1 ^= tg;
+                x = (x - (y & odd)) >> 1;
+                f0 -= f1 & (int64_t)odd, g0 -= g1 & (int64_t)odd;
+                f1 *= 2, g1 *= 2;
+            }
+            uint64_t na[4], nb[4];
+            if (combine(na, a, b, f0, g0)) f0 = -f0, g0 = -g0;
+            if (combine(nb, a, b, f1, g1)) f1 = -f1, g1 = -g1;
+            std::memcpy(a, na, 32);
+            std::memcpy(b, nb, 32);
+            const Fp nu = combine_mod(u, w, f0, g0);
+            w = combine_mod(u, w, f1, g1);
+            u = nu;
+        }
+        // w = 2^(17 (31 - 64)) / this; times 2^(768 + 17 * 33) / 2^256 is 2^512 / this
+        static const Fp undo = [] {
+            Fp t = one();   // 2^256
+            for (int i = 0; i < 512 + 17 * 33; ++i) t = t + t;
+            return t;
+        }();
+        return w * undo;
     }
+
+private:
+    // r = |f a + g b| / 2^31 (an exact division), true when the sum was negative
+    static bool combine(uint64_t r[4], const uint64_t a[4], const uint64_t b[4], int64_t f, int64_t g) {
+        uint64_t t[5];
+        __int128 c = 0;
+        for (int i = 0; i < 4; ++i) {   // |f|, |g| <= 2^31: the sum of both products and the carry fits
+            c += (__int128)f * a[i] + (__int128)g * b[i];
+            t[i] = (uint64_t)c;
+            c >>= 64;
+        }
+        t[4] = (uint64_t)c;
+        const uint64_t neg = 0 - (t[4] >> 63);
+        u128 d = neg & 1;
+        for (int i = 0; i < 5; ++i) { d += t[i] ^ neg; t[i] = (uint64_t)d; d >>= 64; }
+        for (int i = 0; i < 4; ++i) r[i] = (t[i] >> 31) | (t[i + 1] << 33);
+        return neg;
+    }
+    // (f u + g w) / 2^64 modulo p
+    static Fp combine_mod(const Fp& u, const Fp& w, int64_t f, int64_t g) {
+        const Fp x = f < 0 ? u.neg() : u, y = g < 0 ? w.neg() : w;
+        const uint64_t m0 = f < 0 ? 0 - (uint64_t)f : (uint64_t)f, m1 = g < 0 ? 0 - (uint64_t)g : (uint64_t)g;
+        uint64_t t[5];
+        u128 c = 0;
+        for (int i = 0; i < 4; ++i) { c += (u128)m0 * x.v[i] + (u128)m1 * y.v[i]; t[i] = (uint64_t)c; c >>= 64; }
+        t[4] = (uint64_t)c;
+        const uint64_t m = t[0] * P.inv;
+        c = ((u128)m * P.p[0] + t[0]) >> 64;
+        for (int i = 1; i < 4; ++i) { c += (u128)m * P.p[i] + t[i]; t[i - 1] = (uint64_t)c; c >>= 64; }
+        t[3] = (uint64_t)(c + t[4]);
+        return reduced(t[0], t[1], t[2], t[3]);
+    }
+
+public:
     void canonical(uint64_t out[4]) const {   // leave Montgomery form
         Fp one_raw{{1, 0, 0, 0}};
         Fp r = *this * one_raw;
@@ -135,6 +235,24 @@ struct Xyzz {
         F X3 = M.sqr() - S.dbl();
         F Y3 = M * (S - X3) - W * Y;
         return {X3, Y3, V * ZZ, W * ZZZ};
+    }
+    // 2^k times this. The doublings run on Jacobian coordinates, 7 products
+    // each against 9 (dbl-2009-l, a = 0; 0.80 against 0.87 us on Fq2, within 5 % on Fq,
+    // where the chain of three products bounds both): (X ZZ, Y ZZZ, ZZ) is the same point
+    // with Z = ZZ, since ZZ^3 = ZZZ^2, and (X, Y, Z^2, Z^3) leads back.
+    Xyzz dbl_n(unsigned k) const {
+        if (is_inf() || k == 0) return *this;
+        if (k == 1) return dbl();
+        F x = X * ZZ, y = Y * ZZZ, z = ZZ;
+        for (; k; --k) {
+            const F A = x.sqr(), B = y.sqr(), C = B.sqr();
+            const F D = (x * B).dbl().dbl(), E = A.dbl() + A;
+            z = (y * z).dbl();
+            x = E.sqr() - D.dbl();
+            y = E * (D - x) - C.dbl().dbl().dbl();
+        }
+        const F zz = z.sqr();
+        return {x, y, zz, zz * z};
     }
     Xyzz add(const Xyzz& o) const {
         if (o.is_inf()) return *this;

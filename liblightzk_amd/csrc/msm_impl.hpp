@@ -635,6 +635,7 @@ struct MsmBatchLayout {
     std::vector<uint32_t> conv_of;     // instance -> task
     uint64_t conv_total = 0;
     size_t o_conv = 0, o_convdesc = 0;
+    size_t o_upload_end = 0, o_download_end = 0;
 };
 
 template <class F>
@@ -730,26 +731,6 @@ static MsmBatchLayout msm_layout(hzk_ctx* ctx, const MsmJob* jobs, size_t count)
         if (lv > L.hot_levels) L.hot_levels = lv;
     }
     for (int s = 0; s < SP_COUNT; ++s) L.tot[s] = L.begin[(size_t)s * (count + 1) + count];
-    size_t off = 0;
-    auto take = [&off](size_t bytes) { size_t o = (off + 255) & ~size_t(255); off = o + bytes; return o; };
-    L.o_inst = take(count * sizeof(MsmInst));
-    L.o_begin = take(L.begin.size() * 8);
-    L.o_stats = take(count * 16);
-    L.o_digits = take(L.tot[SP_ENTRY] * 4);
-    L.o_count = take(L.tot[SP_CNT] * 4);
-    L.o_tiles = take(L.tot[SP_SCANTILE] * 8);
-    L.o_sub = take(L.tot[SP_GROUP] * 4);
-    L.o_rows = take(L.tot[SP_ROW] * 4);
-    L.o_cidx = take(L.two_level ? L.tot[SP_ENTRY] * 4 : 0);
-    L.o_ckey = take(L.unpacked ? L.tot[SP_ENTRY] * 2 : 0);
-    L.o_offs = take(L.tot[SP_KEY] * 4);
-    L.o_sorted = take(L.tot[SP_ENTRY] * 4);
-    const size_t raw = (size_t)raw_vec<F>() * 16;   // bytes per raw accumulator state
-    L.o_chunk2key = take(L.tot[SP_CHUNK] * 4);
-    L.o_bucket = take(L.tot[SP_KEY] * raw);
-    L.o_carry = take(2 * L.tot[SP_CHUNK] * raw);             // head and tail partial per chunk
-    L.o_tsum = take(L.tot[SP_BRED] * raw);                   // window values (device-side combine)
-    L.o_win = take(2 * L.tot[SP_WIN] * sizeof(xyzz_t<F>));   // P_p, RS_p per part (R = 2^256 points, for the host)
     {
         std::map<const void*, uint64_t> need;   // source array -> points referenced (virtual points of level tables)
         for (size_t i = 0; i < count; ++i)
@@ -765,9 +746,33 @@ static MsmBatchLayout msm_layout(hzk_ctx* ctx, const MsmJob* jobs, size_t count)
         L.conv_of.assign(count, UINT32_MAX);   // UINT32_MAX: bases already converted
         for (size_t i = 0; i < count; ++i)
             if (jobs[i].form == 0) L.conv_of[i] = task_of[L.inst[i].bases];
-        L.o_conv = take(pts * (g2 ? 128 : 64));
-        L.o_convdesc = take(L.conv.size() * sizeof(MsmConvTask));
     }
+    size_t off = 0;
+    auto take = [&off](size_t bytes) { size_t o = (off + 255) & ~size_t(255); off = o + bytes; return o; };
+    // descriptors, uploaded in one copy (o_inst .. o_upload_end)
+    L.o_inst = take(count * sizeof(MsmInst));
+    L.o_begin = take(L.begin.size() * 8);
+    L.o_convdesc = take(L.conv.size() * sizeof(MsmConvTask));
+    L.o_upload_end = off;
+    L.o_digits = take(L.tot[SP_ENTRY] * 4);
+    L.o_count = take(L.tot[SP_CNT] * 4);
+    L.o_tiles = take(L.tot[SP_SCANTILE] * 8);
+    L.o_sub = take(L.tot[SP_GROUP] * 4);
+    L.o_rows = take(L.tot[SP_ROW] * 4);
+    L.o_cidx = take(L.two_level ? L.tot[SP_ENTRY] * 4 : 0);
+    L.o_ckey = take(L.unpacked ? L.tot[SP_ENTRY] * 2 : 0);
+    L.o_offs = take(L.tot[SP_KEY] * 4);
+    L.o_sorted = take(L.tot[SP_ENTRY] * 4);
+    const size_t raw = (size_t)raw_vec<F>() * 16;   // bytes per raw accumulator state
+    L.o_chunk2key = take(L.tot[SP_CHUNK] * 4);
+    L.o_bucket = take(L.tot[SP_KEY] * raw);
+    L.o_carry = take(2 * L.tot[SP_CHUNK] * raw);             // head and tail partial per chunk
+    L.o_tsum = take(L.tot[SP_BRED] * raw);                   // window values (device-side combine)
+    // results for the host, downloaded in one copy (o_stats .. o_download_end)
+    L.o_stats = take(count * 16);
+    L.o_win = take(2 * L.tot[SP_WIN] * sizeof(xyzz_t<F>));   // P_p, RS_p per part (R = 2^256 points, for the host)
+    L.o_download_end = off;
+    L.o_conv = take(L.conv_total * (g2 ? 128 : 64));
     L.bytes = off + 256;
     return L;
 }
@@ -903,9 +908,11 @@ int msm_batch_run(hzk_ctx* ctx, const MsmJob* jobs, size_t count, int dests_on_h
         rc = ensure_scratch(ctx, L.bytes);
         if (rc) return rc;
     }
-    const size_t conv_bytes = L.conv.size() * sizeof(MsmConvTask);
-    const size_t host_bytes = count * sizeof(MsmInst) + L.begin.size() * 8 + 2 * L.tot[SP_WIN] * sizeof(xyzz_t<F>) + count * 16 +
-                              conv_bytes + 1024;
+    // staging: the descriptors as they lie in the scratch, the downloaded
+    // window sums and statistics, the results
+    const size_t up_bytes = L.o_upload_end - L.o_inst, down_bytes = L.o_download_end - L.o_stats;
+    const size_t s_down = (up_bytes + 255) & ~size_t(255), s_out = (s_down + down_bytes + 255) & ~size_t(255);
+    const size_t host_bytes = s_out + count * 3 * sizeof(F);
     char* pin;
     int slot = -1;
     std::vector<char> pageable;
@@ -924,14 +931,9 @@ int msm_batch_run(hzk_ctx* ctx, const MsmJob* jobs, size_t count, int dests_on_h
         if (L.conv_of[i] != UINT32_MAX) L.inst[i].bases = L.conv[L.conv_of[i]].dst;
     // descriptors and work-space starts
     std::memcpy(pin, L.inst.data(), count * sizeof(MsmInst));
-    std::memcpy(pin + count * sizeof(MsmInst), L.begin.data(), L.begin.size() * 8);
-    HZK_HIP(ctx, hipMemcpyAsync(base + L.o_inst, pin, count * sizeof(MsmInst), hipMemcpyHostToDevice, st));
-    HZK_HIP(ctx, hipMemcpyAsync(base + L.o_begin, pin + count * sizeof(MsmInst), L.begin.size() * 8, hipMemcpyHostToDevice, st));
-    char* pconv = pin + count * sizeof(MsmInst) + L.begin.size() * 8 + 2 * L.tot[SP_WIN] * sizeof(xyzz_t<F>) + count * 16;
-    if (conv_bytes) {
-        std::memcpy(pconv, L.conv.data(), conv_bytes);
-        HZK_HIP(ctx, hipMemcpyAsync(base + L.o_convdesc, pconv, conv_bytes, hipMemcpyHostToDevice, st));
-    }
+    std::memcpy(pin + (L.o_begin - L.o_inst), L.begin.data(), L.begin.size() * 8);
+    if (!L.conv.empty()) std::memcpy(pin + (L.o_convdesc - L.o_inst), L.conv.data(), L.conv.size() * sizeof(MsmConvTask));
+    HZK_HIP(ctx, hipMemcpyAsync(base + L.o_inst, pin, up_bytes, hipMemcpyHostToDevice, st));
 
     if (capture) {
         std::string key = shape_key<F>(L, device_combine != 0);
@@ -964,11 +966,10 @@ int msm_batch_run(hzk_ctx* ctx, const MsmJob* jobs, size_t count, int dests_on_h
         HZK_HIP(ctx, hipStreamSynchronize(st));   // pageable staging (no-alloc scratch): wait for the copies
         return 0;
     }
-    char* hwin = pin + count * sizeof(MsmInst) + L.begin.size() * 8;
-    uint32_t* hstats = (uint32_t*)(hwin + 2 * L.tot[SP_WIN] * sizeof(xyzz_t<F>));
-    HZK_HIP(ctx, hipMemcpyAsync(hwin, base + L.o_win, 2 * L.tot[SP_WIN] * sizeof(xyzz_t<F>), hipMemcpyDeviceToHost, st));
-    HZK_HIP(ctx, hipMemcpyAsync(hstats, base + L.o_stats, count * 16, hipMemcpyDeviceToHost, st));
-    if (slot >= 0) {
+    const uint32_t* hstats = (const uint32_t*)(pin + s_down);
+    const char* hwin = pin + s_down + (L.o_win - L.o_stats);
+    HZK_HIP(ctx, hipMemcpyAsync(pin + s_down, base + L.o_stats, down_bytes, hipMemcpyDeviceToHost, st));
+    if (slot >= 0) {   // a slot that an error leaves early is free once the download is done
         rc = stage_fence(ctx, slot);
         if (rc) return rc;
     }
@@ -981,7 +982,7 @@ int msm_batch_run(hzk_ctx* ctx, const MsmJob* jobs, size_t count, int dests_on_h
     std::vector<uint64_t> tbeg(count + 1, 0);
     for (size_t i = 0; i < count; ++i) tbeg[i + 1] = tbeg[i] + L.inst[i].W;
     std::vector<HostPt> T(tbeg[count]);
-    parallel_for((long)tbeg[count], [&](long q) {
+    const auto window_value = [&](long q) {
         const size_t i = std::upper_bound(tbeg.begin(), tbeg.end(), (uint64_t)q) - tbeg.begin() - 1;
         const MsmInst& d = L.inst[i];
         const size_t j = (size_t)q - tbeg[i];
@@ -995,21 +996,24 @@ int msm_batch_run(hzk_ctx* ctx, const MsmJob* jobs, size_t count, int dests_on_h
             y = y.add(suf);
         }
         if (d.S > 1) {
-            for (uint32_t k = 1; k < d.G / d.S * d.g; k <<= 1) y = y.dbl();
-            acc = acc.add(y);
+            uint32_t k = 0;
+            while ((1u << k) < d.G / d.S * d.g) ++k;
+            acc = acc.add(y.dbl_n(k));
         }
         T[q] = acc;
-    });
+    };
+    // a window of one part is only read: nothing to wake the pool for
+    if (L.tot[SP_WIN] == tbeg[count]) for (long q = 0; q < (long)tbeg[count]; ++q) window_value(q);
+    else parallel_for((long)tbeg[count], window_value);
     // Horner over windows, instances in parallel
-    std::vector<char> out(count * 3 * sizeof(F));
+    char* const out = pin + s_out;   // pinned: a copy from pageable memory goes through a staging copy and a wait of its own
     parallel_for((long)count, [&](long i) {
         const MsmInst& d = L.inst[i];
         HostPt acc = HostPt::inf();
         for (int j = (int)d.W - 1; j >= 0; --j) {
             // a bucket set spans Lg digit windows of c bits; plain windows are wb or wb + 1 bits
             const uint32_t shift = d.Lg > 1 ? d.c * d.Lg : d.wb + ((uint32_t)j < d.wx ? 1u : 0u);
-            for (uint32_t q = 0; q < shift; ++q) acc = acc.dbl();
-            acc = acc.add(T[tbeg[i] + j]);
+            acc = acc.dbl_n(shift).add(T[tbeg[i] + j]);
         }
         acc.store_jacobian(&out[i * 3 * sizeof(F)]);
     });
