@@ -55,7 +55,7 @@ enum MsmSpace {
     SP_SMALL,       // one workgroup per window of a small instance
     SP_KEY,         // nk + 1 entries per instance (offsets, bucket sums)
     SP_CHUNK,       // accumulation chunks of K sorted entries (upper bound)
-    SP_BRED,        // window values (device-side combine)
+    SP_BRED,        // windows (two result points each)
     SP_WIN,         // window-sum partials (S per window)
     SP_ENTRY,       // n * W digit / sorted-entry slots
     SP_COUNT

@@ -416,6 +416,13 @@ __global__ void __launch_bounds__(256) k_msm_fixup(MsmBatchDev b, const uint32_t
     acc.store_raw(bucket + (size_t)RW * (kb + k));
 }
 
+// log2 of the buckets of a part where a window has several, else 0
+__host__ __device__ inline uint32_t window_part_log(const MsmInst& d) {
+    uint32_t k = 0;
+    if (d.S > 1) while ((1u << k) < d.NB / d.S) ++k;
+    return k;
+}
+
 // ------------------------------------------------------------------ 7. bucket reduction
 // A window's value is sum_{d=1..NB} d * B_d. Workgroup per (window, part of
 // NB / S buckets), each lane group (slot) of it takes the g consecutive
@@ -424,14 +431,14 @@ __global__ void __launch_bounds__(256) k_msm_fixup(MsmBatchDev b, const uint32_t
 // value, weights relative to its first bucket, is
 //     sum_t [ A_t + g * t * R_t ] = sum_t A_t + g * sum_{t>=1} X_t,
 // X_t the suffix sums of R, one LDS scan. Each part yields its value P_p and
-// its bucket sum RS_p; the host adds p * (NB / S) * RS_p. Buckets and LDS slots
-// hold raw accumulator states; only P_p and RS_p are converted to R = 2^256
-// XYZZ points for the host.
+// its bucket sum RS_p; the window is sum_p P_p + (NB / S) * sum_p p RS_p. Both
+// sums (k_window_value) leave as R = 2^256 XYZZ points; the factor is applied
+// among the doublings between windows.
 // T = 256 threads for single MSMs, 64 in wide batches (fewer scan and tree
 // steps per bucket; the batch fills the GPU by itself).
 template <class F, int T>
 __global__ void __launch_bounds__(T) k_window_sum(MsmBatchDev b, const uint32_t* __restrict__ bucket, const uint32_t* __restrict__ offs,
-                                                  xyzz_t<F>* __restrict__ winsum) {
+                                                  uint32_t* __restrict__ parts, xyzz_t<F>* __restrict__ wval) {
     using A = LanePoint<F>;
     using S = LdsLanes<F, T>;
     constexpr int RW = A::RAW_WORDS;
@@ -472,59 +479,65 @@ __global__ void __launch_bounds__(T) k_window_sum(MsmBatchDev b, const uint32_t*
         __syncthreads();
         if (slot + off < n) run.add(sh.get(off));
     }
+    uint32_t* out = parts + (size_t)RW * 2 * blockIdx.x;   // P_p, RS_p
     if (slot == 0) {
-        run.store_xyzz(winsum + 2 * blockIdx.x + 1);   // RS_p
+        if (d.S > 1) run.store_raw(out + RW);
         run.set_inf();
     }
     for (uint32_t k = 1; k < m; k <<= 1) run.dbl();
     a.add(run);
     sh.tree_sum(a, n);
-    if (slot == 0) a.store_xyzz(winsum + 2 * blockIdx.x);   // P_p
+    if (slot == 0) {
+        if (d.S > 1) a.store_raw(out);
+        else a.store_xyzz(wval + 2 * (space_g(b, SP_BRED)[ii] + j));
+    }
+}
+
+// The parts of a window as two points, workgroup per window: sum_p P_p and
+// sum_p p RS_p (the suffix sums of RS over p >= 1, summed). S slots scan RS
+// while S others sum P in the same steps, then a tree: 2 log2 S additions one
+// after the other, 31 us at 32 parts of G1 and 76 us at 64 parts of G2. The
+// host's 3 S additions a window, shared by a worker pool, with a copy of 2 S
+// points took longer: 2^16 points 559 -> 506 us, 200003 of G2 1705 -> 1500,
+// 32 G1 MSMs of a batch 3754 -> 3500.
+template <class F>
+constexpr int WINDOW_VALUE_T = 128 * LanePoint<F>::LANES;   // 2 x 64 parts
+template <class F>
+__global__ void __launch_bounds__(WINDOW_VALUE_T<F>) k_window_value(MsmBatchDev b, const uint32_t* __restrict__ parts,
+                                                                    xyzz_t<F>* __restrict__ wval) {
+    using A = LanePoint<F>;
+    constexpr int RW = A::RAW_WORDS;
+    __shared__ uint32_t shw[LdsLanes<F, WINDOW_VALUE_T<F>>::WORDS];
+    const LdsLanes<F, WINDOW_VALUE_T<F>> sh{shw};
+    const uint64_t* vbeg = space_g(b, SP_BRED);
+    const uint32_t ii = find_inst_g(vbeg, b.ninst, blockIdx.x);
+    const MsmInst& d = b.inst[ii];
+    const uint32_t S = d.S, j = (uint32_t)(blockIdx.x - vbeg[ii]);
+    if (S == 1) return;   // written by k_window_sum
+    const uint32_t slot = threadIdx.x / A::LANES;
+    const bool sums = slot >= S;               // the half that sums P
+    const uint32_t p = sums ? slot - S : slot;
+    A x;
+    x.set_inf();
+    if (p < S) x = A::load_raw(parts + (size_t)RW * (2 * (space_g(b, SP_WIN)[ii] + (size_t)j * S + p) + (sums ? 0 : 1)));
+    for (uint32_t off = 1; off < S; off <<= 1) {
+        const uint32_t step = sums ? S / 2 / off : off;
+        __syncthreads();
+        sh.put(x);
+        __syncthreads();
+        if (sums ? p < step : p + step < S) x.add(sh.get(step));
+    }
+    if (slot == S) x.store_xyzz(wval + 2 * blockIdx.x);
+    if (slot == 0) x.set_inf();
+    sh.tree_sum(x, S);
+    if (slot == 0) x.store_xyzz(wval + 2 * blockIdx.x + 1);
 }
 
 // ------------------------------------------------------------------ 8. device-side combine (optional)
-// The host's combine as two kernels, in the 29-bit accumulator arithmetic.
-// k_msm_combine_windows: workgroup per (instance, window), lane per part p:
-// T_j = sum_p P_p + (g Gs) sum_p p RS_p, the last sum as the sum over p >= 1
-// of the suffix sums of RS (an LDS scan), stored as a raw state. k_msm_combine_horner: lane
+// The host's combine as a kernel, in the 29-bit accumulator arithmetic: lane
 // per instance, Horner over the windows (the dependent doublings that make
-// this path slower than the host's), then the normalised Jacobian
-// (x, y, 1) or (0, 1, 0): the bytes the host writes.
-// Per-thread accumulator slots in LDS, word-major: word w of slot t at
-// sh[w * T + t], so the lanes of a wave touch consecutive words (a point per
-// slot in a row would put every lane's word w in the same bank)
-template <class F, int T>
-struct LdsPoints {
-    using A = acc29_t<F>;
-    static constexpr int W = A::RAW_WORDS;
-    uint32_t* sh;
-    HZK_DEV void put(uint32_t t, const A& p) const {
-        uint32_t w[W];
-        p.to_words(w);
-#pragma unroll
-        for (int i = 0; i < W; ++i) sh[i * T + t] = w[i];
-    }
-    HZK_DEV A get(uint32_t t) const {
-        uint32_t w[W];
-#pragma unroll
-        for (int i = 0; i < W; ++i) w[i] = sh[i * T + t];
-        return A::from_words(w);
-    }
-};
-
-// tree sum of slots 0..T) into slot 0
-template <class F, int T>
-HZK_DEV void lds_tree_sum(const LdsPoints<F, T>& sh, uint32_t t) {
-    for (uint32_t off = T / 2; off > 0; off >>= 1) {
-        if (t < off) {
-            auto x = sh.get(t);
-            x.add(sh.get(t + off));
-            sh.put(t, x);
-        }
-        __syncthreads();
-    }
-}
-
+// this path slower than the host's), then the normalised Jacobian (x, y, 1) or
+// (0, 1, 0): the bytes the host writes.
 template <class F>
 HZK_DEV acc29_t<F> acc_from_xyzz(const xyzz_t<F>& p);
 template <>
@@ -542,66 +555,21 @@ HZK_DEV g2acc29 acc_from_xyzz<fq2_t>(const xyzz_t<fq2_t>& p) {
 }
 
 template <class F>
-__global__ void __launch_bounds__(64) k_msm_combine_windows(MsmBatchDev b, const xyzz_t<F>* __restrict__ win, uint32_t maxw,
-                                                            uint4* __restrict__ tsum) {
+__global__ void __launch_bounds__(64) k_msm_combine_horner(MsmBatchDev b, const xyzz_t<F>* __restrict__ wval) {
     using A = acc29_t<F>;
-    constexpr int RW = raw_vec<F>();
-    __shared__ uint32_t shw[LdsPoints<F, 64>::W * 64];
-    const LdsPoints<F, 64> sh{shw};
-    const uint32_t i = blockIdx.x / maxw, j = blockIdx.x % maxw, t = threadIdx.x;
-    const MsmInst& d = b.inst[i];
-    if (j >= d.W) return;   // uniform per workgroup
-    const xyzz_t<F>* pj = win + 2 * (space_g(b, SP_WIN)[i] + (size_t)j * d.S);
-    A P, RS;
-    P.set_inf();
-    RS.set_inf();
-    if (t < d.S) {
-        P = acc_from_xyzz<F>(pj[2 * t]);
-        RS = acc_from_xyzz<F>(pj[2 * t + 1]);
-    }
-    // inclusive suffix scan of RS: slot t = sum_{p >= t} RS_p
-    sh.put(t, RS);
-    __syncthreads();
-    for (uint32_t off = 1; off < 64; off <<= 1) {
-        A x = sh.get(t);
-        if (t + off < 64) x.add(sh.get(t + off));
-        __syncthreads();
-        sh.put(t, x);
-        __syncthreads();
-    }
-    A y = sh.get(t);
-    if (t == 0) y.set_inf();   // sum_p p RS_p = sum_{t >= 1} slot t
-    __syncthreads();
-    sh.put(t, y);
-    __syncthreads();
-    lds_tree_sum<F, 64>(sh, t);
-    A ysum = sh.get(0);
-    __syncthreads();
-    sh.put(t, P);
-    __syncthreads();
-    lds_tree_sum<F, 64>(sh, t);
-    if (t == 0) {
-        A T = sh.get(0);
-        for (uint32_t k = 1; k < d.G / d.S * d.g; k <<= 1) ysum.dbl();
-        T.add(ysum);
-        T.store_raw(tsum + (size_t)RW * (space_g(b, SP_BRED)[i] + j));
-    }
-}
-
-template <class F>
-__global__ void __launch_bounds__(64) k_msm_combine_horner(MsmBatchDev b, const uint4* __restrict__ tsum) {
-    using A = acc29_t<F>;
-    constexpr int RW = raw_vec<F>();
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= b.ninst) return;
     const MsmInst& d = b.inst[i];
-    const uint4* T = tsum + (size_t)RW * space_g(b, SP_BRED)[i];
+    const xyzz_t<F>* v = wval + 2 * space_g(b, SP_BRED)[i];
+    const uint32_t k = window_part_log(d);
     A acc;
     acc.set_inf();
     for (int j = (int)d.W - 1; j >= 0; --j) {
         const uint32_t shift = d.Lg > 1 ? d.c * d.Lg : d.wb + ((uint32_t)j < d.wx ? 1u : 0u);
-        for (uint32_t q = 0; q < shift; ++q) acc.dbl();
-        acc.add(A::load_raw(T + (size_t)RW * j));
+        for (uint32_t q = k; q < shift; ++q) acc.dbl();
+        if (d.S > 1) acc.add(acc_from_xyzz<F>(v[2 * j + 1]));
+        for (uint32_t q = 0; q < k; ++q) acc.dbl();
+        acc.add(acc_from_xyzz<F>(v[2 * j]));
     }
     const xyzz_t<F> r = acc.to_xyzz();
     F* out = (F*)d.dest;
@@ -621,6 +589,7 @@ struct MsmBatchLayout {
     std::vector<uint64_t> begin;   // [SP_COUNT][ninst + 1]
     uint64_t tot[SP_COUNT];
     MsmSortMax sort_max;
+    uint32_t max_parts = 1;        // parts per window
     uint32_t hot_levels = 0;       // levels of k_msm_hot_sum (upper bound)
     bool two_level = false;        // some instance is sorted in two levels
     bool unpacked = false;         // some coarse entries take two arrays
@@ -628,7 +597,7 @@ struct MsmBatchLayout {
     size_t bytes = 0;              // scratch needed
     // scratch offsets
     size_t o_inst, o_begin, o_stats, o_digits, o_count, o_tiles, o_sub, o_rows, o_cidx, o_ckey, o_offs, o_sorted, o_chunk2key, o_bucket,
-        o_carry, o_tsum, o_win;
+        o_carry, o_parts, o_wval;
     // base arrays converted for the accumulation, one per distinct source
     // array (its largest referenced point count), and which one each instance reads
     std::vector<MsmConvTask> conv;     // dst holds the offset into the scratch until run time
@@ -695,6 +664,7 @@ static MsmBatchLayout msm_layout(hzk_ctx* ctx, const MsmJob* jobs, size_t count)
         const uint32_t slots = regime == MSM_REGIME_BATCH ? LdsLanes<F, 64>::SLOTS : LdsLanes<F, 256>::SLOTS;
         d.S = 1;
         while (d.S < 64 && d.G / d.S > slots) d.S *= 2;
+        L.max_parts = std::max(L.max_parts, d.S);
         d.T = msm_tiles(d.nd);
         d.tile = (d.nd + d.T - 1) / d.T;
         d.small = d.n <= (regime == MSM_REGIME_BATCH ? MSM_SMALL_BATCH_N : MSM_SMALL_N) && d.NB <= MSM_SMALL_NB;
@@ -767,10 +737,10 @@ static MsmBatchLayout msm_layout(hzk_ctx* ctx, const MsmJob* jobs, size_t count)
     L.o_chunk2key = take(L.tot[SP_CHUNK] * 4);
     L.o_bucket = take(L.tot[SP_KEY] * raw);
     L.o_carry = take(2 * L.tot[SP_CHUNK] * raw);             // head and tail partial per chunk
-    L.o_tsum = take(L.tot[SP_BRED] * raw);                   // window values (device-side combine)
+    L.o_parts = take(2 * L.tot[SP_WIN] * raw);               // P_p, RS_p per part of a window
     // results for the host, downloaded in one copy (o_stats .. o_download_end)
     L.o_stats = take(count * 16);
-    L.o_win = take(2 * L.tot[SP_WIN] * sizeof(xyzz_t<F>));   // P_p, RS_p per part (R = 2^256 points, for the host)
+    L.o_wval = take(2 * L.tot[SP_BRED] * sizeof(xyzz_t<F>));   // two points per window (R = 2^256, for the host)
     L.o_download_end = off;
     L.o_conv = take(L.conv_total * (g2 ? 128 : 64));
     L.bytes = off + 256;
@@ -799,7 +769,8 @@ static void msm_device_stages(hzk_ctx* ctx, const MsmBatchLayout& L, char* base)
     uint32_t* chunk2key = (uint32_t*)(base + L.o_chunk2key);
     uint4* bucket = (uint4*)(base + L.o_bucket);
     uint4* carry = (uint4*)(base + L.o_carry);
-    xyzz_t<F>* win = (xyzz_t<F>*)(base + L.o_win);
+    uint32_t* parts = (uint32_t*)(base + L.o_parts);
+    xyzz_t<F>* wval = (xyzz_t<F>*)(base + L.o_wval);
     hipStream_t st = ctx->stream;
 
     if (L.conv_total) {
@@ -838,10 +809,13 @@ static void msm_device_stages(hzk_ctx* ctx, const MsmBatchLayout& L, char* base)
         TimedLaunch tl(ctx, "msm_bucket_reduce");
         if (L.regime == MSM_REGIME_BATCH)
             hipLaunchKernelGGL((k_window_sum<F, 64>), dim3((unsigned)L.tot[SP_WIN]), dim3(64), 0, st, b, (const uint32_t*)bucket,
-                               (const uint32_t*)sb.offs, win);
+                               (const uint32_t*)sb.offs, parts, wval);
         else
             hipLaunchKernelGGL((k_window_sum<F, 256>), dim3((unsigned)L.tot[SP_WIN]), dim3(256), 0, st, b, (const uint32_t*)bucket,
-                               (const uint32_t*)sb.offs, win);
+                               (const uint32_t*)sb.offs, parts, wval);
+        if (L.max_parts > 1)
+            hipLaunchKernelGGL(k_window_value<F>, dim3((unsigned)L.tot[SP_BRED]),
+                               dim3(std::max<unsigned>(64, 2 * L.max_parts * LanePoint<F>::LANES)), 0, st, b, (const uint32_t*)parts, wval);
     }
 }
 
@@ -852,14 +826,9 @@ static void msm_launch_combine(hzk_ctx* ctx, const MsmBatchLayout& L, char* base
     b.begin = (const uint64_t*)(base + L.o_begin);
     b.ninst = (uint32_t)L.inst.size();
     b.stats = (uint32_t*)(base + L.o_stats);
-    uint32_t maxw = 1;
-    for (const MsmInst& d : L.inst) maxw = std::max(maxw, d.W);
-    uint4* tsum = (uint4*)(base + L.o_tsum);
     TimedLaunch tl(ctx, "msm_combine");
-    hipLaunchKernelGGL(k_msm_combine_windows<F>, dim3((unsigned)(L.inst.size() * maxw)), dim3(64), 0, ctx->stream, b,
-                       (const xyzz_t<F>*)(base + L.o_win), maxw, tsum);
     hipLaunchKernelGGL(k_msm_combine_horner<F>, dim3(blocks_for(L.inst.size(), 64)), dim3(64), 0, ctx->stream, b,
-                       (const uint4*)tsum);
+                       (const xyzz_t<F>*)(base + L.o_wval));
 }
 
 template <class F>
@@ -967,7 +936,7 @@ int msm_batch_run(hzk_ctx* ctx, const MsmJob* jobs, size_t count, int dests_on_h
         return 0;
     }
     const uint32_t* hstats = (const uint32_t*)(pin + s_down);
-    const char* hwin = pin + s_down + (L.o_win - L.o_stats);
+    const char* hval = pin + s_down + (L.o_wval - L.o_stats);
     HZK_HIP(ctx, hipMemcpyAsync(pin + s_down, base + L.o_stats, down_bytes, hipMemcpyDeviceToHost, st));
     if (slot >= 0) {   // a slot that an error leaves early is free once the download is done
         rc = stage_fence(ctx, slot);
@@ -975,45 +944,22 @@ int msm_batch_run(hzk_ctx* ctx, const MsmJob* jobs, size_t count, int dests_on_h
     }
     HZK_HIP(ctx, hipStreamSynchronize(st));
 
-    // window values on the host, all (instance, window) pairs in parallel:
-    // T_j = sum_p P_p + (g Gs) * sum_p p RS_p, the last sum as the sum of the
-    // suffix sums of RS over p >= 1
-    const uint64_t* wbeg = L.begin.data() + (size_t)SP_WIN * (count + 1);
-    std::vector<uint64_t> tbeg(count + 1, 0);
-    for (size_t i = 0; i < count; ++i) tbeg[i + 1] = tbeg[i] + L.inst[i].W;
-    std::vector<HostPt> T(tbeg[count]);
-    const auto window_value = [&](long q) {
-        const size_t i = std::upper_bound(tbeg.begin(), tbeg.end(), (uint64_t)q) - tbeg.begin() - 1;
-        const MsmInst& d = L.inst[i];
-        const size_t j = (size_t)q - tbeg[i];
-        auto pt = [&](uint32_t p, int which) {
-            return HostPt::load_xyzz(hwin + (2 * (wbeg[i] + j * d.S + p) + which) * sizeof(xyzz_t<F>));
-        };
-        HostPt acc = HostPt::inf(), suf = HostPt::inf(), y = HostPt::inf();
-        for (uint32_t p = 0; p < d.S; ++p) acc = acc.add(pt(p, 0));
-        for (uint32_t p = d.S - 1; p >= 1; --p) {
-            suf = suf.add(pt(p, 1));
-            y = y.add(suf);
-        }
-        if (d.S > 1) {
-            uint32_t k = 0;
-            while ((1u << k) < d.G / d.S * d.g) ++k;
-            acc = acc.add(y.dbl_n(k));
-        }
-        T[q] = acc;
-    };
-    // a window of one part is only read: nothing to wake the pool for
-    if (L.tot[SP_WIN] == tbeg[count]) for (long q = 0; q < (long)tbeg[count]; ++q) window_value(q);
-    else parallel_for((long)tbeg[count], window_value);
     // Horner over windows, instances in parallel
     char* const out = pin + s_out;   // pinned: a copy from pageable memory goes through a staging copy and a wait of its own
+    const uint64_t* vbeg = L.begin.data() + (size_t)SP_BRED * (count + 1);
     parallel_for((long)count, [&](long i) {
         const MsmInst& d = L.inst[i];
+        const uint32_t k = window_part_log(d);
         HostPt acc = HostPt::inf();
         for (int j = (int)d.W - 1; j >= 0; --j) {
-            // a bucket set spans Lg digit windows of c bits; plain windows are wb or wb + 1 bits
+            // a window is sum_p P_p + 2^k sum_p p RS_p: the second sum joins k
+            // doublings early. A bucket set spans Lg digit windows of c bits;
+            // plain windows are wb or wb + 1 bits, either more than k
+            const char* v = hval + 2 * (vbeg[i] + j) * sizeof(xyzz_t<F>);
             const uint32_t shift = d.Lg > 1 ? d.c * d.Lg : d.wb + ((uint32_t)j < d.wx ? 1u : 0u);
-            acc = acc.dbl_n(shift).add(T[tbeg[i] + j]);
+            acc = acc.dbl_n(shift - k);
+            if (d.S > 1) acc = acc.add(HostPt::load_xyzz(v + sizeof(xyzz_t<F>)));
+            acc = acc.dbl_n(k).add(HostPt::load_xyzz(v));
         }
         acc.store_jacobian(&out[i * 3 * sizeof(F)]);
     });

@@ -65,3 +65,23 @@ def test_run_lengths(ctx, orc, group, regime, c):
     finally:
         set_plan(group, log_n, 0)
         ctx.set_msm_regime(-1)
+
+
+# parts of a window: 64 (the most) down to 1 as g grows; sparse windows leave most parts empty
+@pytest.mark.parametrize("group", [1, 2])
+@pytest.mark.parametrize("regime", [0, 1])
+@pytest.mark.parametrize("n", [3, 6000])
+def test_window_parts(ctx, orc, group, regime, n):
+    s, k = orc.gen_fr(23, 0, n), orc.gen_fr(23, 1, n)
+    bases = (orc.g1_mul_gen if group == 1 else orc.g2_mul_gen)(k)
+    want = orc.msm_closed_form(s, k, group)
+    log_n = n.bit_length() - 1
+    set_plan = ctx.msm_tune_set if regime == 0 else ctx.msm_batch_tune_set
+    ctx.set_msm_regime(regime)
+    try:
+        for g in (1 << i for i in range(12)):
+            set_plan(group, log_n, 13, 8, g)
+            assert np.array_equal(_run(ctx, group, s, bases, n), want), g
+    finally:
+        set_plan(group, log_n, 0)
+        ctx.set_msm_regime(-1)
