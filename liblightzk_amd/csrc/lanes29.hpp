@@ -120,6 +120,15 @@ struct LanePoint {
         ((fq_t*)out)[L::elem()] = r;
     }
 
+    // the point of the group that lane `lane` (this one's place in it) belongs to
+    HZK_DEV LanePoint from_lane(int lane) const {
+        LanePoint p;
+#pragma unroll
+        for (int i = 0; i < 9; ++i) p.v.l[i] = __shfl(v.l[i], lane);
+        p.inf = __shfl((int)inf, lane) != 0;
+        return p;
+    }
+
     // this += q (add-2008-s), every special case handled as in g1acc29::add
     HZK_DEV void add(const LanePoint& q) {
         const bool live = !inf && !q.inf;

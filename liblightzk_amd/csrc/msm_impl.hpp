@@ -16,7 +16,7 @@
 
 namespace hzk {
 
-static constexpr uint32_t HOT = 16;         // a bucket spanning more chunks than this is summed by k_msm_hot_sum first
+static constexpr uint32_t HOT = 64;         // a bucket spanning more chunks than this is summed by k_msm_hot_sum first
 static constexpr uint32_t HOT_LIST = 256;   // hot instances a hot-sum block lists in LDS
 
 HZK_DEV uint32_t find_inst_g(const uint64_t* __restrict__ beg, uint32_t ninst, uint64_t gid) {
@@ -407,34 +407,92 @@ __global__ void __launch_bounds__(256) k_msm_hot_sum(MsmBatchDev b, const uint32
     }
 }
 
-// bucket spanning chunks f..l (f < l): bucket = tail(f) + heads(f+1..l), by
-// the lane group of chunk f+1 (the first chunk that continues it)
-template <class F>
+// Buckets that span chunks f..l (f < l): bucket = tail(f) + heads(f+1..l), a
+// lane group per bucket. The groups are numbered by bucket where there are
+// fewer buckets than chunks and by chunk (the bucket's second one works)
+// otherwise, so that few groups of a wave idle. A group adds its first
+// FIX_OWN heads itself; beyond those its wave sums whole runs together where
+// that takes fewer steps than the longest one alone.
+static constexpr uint32_t FIX_OWN = 4;
+
+template <class F, bool BY_KEY>
 __global__ void __launch_bounds__(256) k_msm_fixup(MsmBatchDev b, const uint32_t* __restrict__ offs,
                                                    const uint32_t* __restrict__ chunk2key, const uint32_t* __restrict__ carry,
                                                    uint32_t* __restrict__ bucket) {
     using A = LanePoint<F>;
-    constexpr int RW = A::RAW_WORDS;
-    const uint64_t* cbeg = space_g(b, SP_CHUNK);
-    const uint64_t gid = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / A::LANES;
-    if (gid >= cbeg[b.ninst]) return;
-    uint32_t ii = find_inst_g(cbeg, b.ninst, gid);
-    const MsmInst& d = b.inst[ii];
-    const uint32_t c = (uint32_t)(gid - cbeg[ii]);
-    if ((uint64_t)c * d.K >= b.stats[4 * ii]) return;
-    const uint64_t kb = space_g(b, SP_KEY)[ii];
-    const uint32_t k = chunk2key[gid], start = offs[kb + k];
-    if (start >= c * d.K) return;   // the chunk's first bucket starts in it
-    const uint32_t f = start / d.K;
-    if (c != f + 1) return;
-    const uint32_t l = (offs[kb + k + 1] - 1) / d.K;
-    const uint32_t* base = carry + (size_t)RW * 2 * cbeg[ii];
-    A acc = A::load_raw(base + (size_t)RW * (2 * f + 1));
-    const uint32_t last = l - f > HOT ? f + 1 : l;   // hot: their sum stands in the first
-    for (uint32_t cc = f + 1; cc <= last; ++cc) acc.add(A::load_raw(base + (size_t)RW * 2 * cc));
-    acc.store_raw(bucket + (size_t)RW * (kb + k));
+    constexpr int RW = A::RAW_WORDS, LANES = A::LANES, GROUPS = 64 / LANES;
+    const uint64_t* beg = space_g(b, BY_KEY ? SP_KEY : SP_CHUNK);
+    const uint64_t gid = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / LANES;
+    A acc;
+    acc.set_inf();
+    uint32_t left = 0;                // heads to add, the next one at head
+    const uint32_t* head = nullptr;
+    uint32_t* dst = nullptr;
+    if (gid < beg[b.ninst]) {
+        const uint32_t ii = find_inst_g(beg, b.ninst, gid), at = (uint32_t)(gid - beg[ii]);
+        const MsmInst& d = b.inst[ii];
+        const uint64_t kb = space_g(b, SP_KEY)[ii];
+        const bool any = BY_KEY ? at < d.nk : (uint64_t)at * d.K < b.stats[4 * ii];
+        if (any) {
+            const uint32_t k = BY_KEY ? at : chunk2key[gid], start = offs[kb + k], end = offs[kb + k + 1];
+            const uint32_t f = start / d.K, l = end > start ? (end - 1) / d.K : f;
+            if (f < l && (BY_KEY || at == f + 1)) {
+                const uint32_t* base = carry + (size_t)RW * 2 * space_g(b, SP_CHUNK)[ii];
+                acc = A::load_raw(base + (size_t)RW * (2 * f + 1));
+                head = base + (size_t)RW * 2 * (f + 1);
+                left = l - f > HOT ? 1 : l - f;   // hot: their sum stands in the first
+                dst = bucket + (size_t)RW * (kb + k);
+            }
+        }
+    }
+    const auto add_own = [&](uint32_t steps) {
+        for (uint32_t i = 0; i < steps; ++i) {
+            A x;
+            if (i < left) x = A::load_raw(head + (size_t)RW * 2 * i);
+            else x.set_inf();
+            acc.add(x);
+        }
+    };
+    uint32_t most = left;
+    for (int m = 32; m >= LANES; m >>= 1) most = max(most, (uint32_t)__shfl_xor((int)most, m));
+    if (most == 0) return;   // the whole wave
+    add_own(min(most, FIX_OWN));
+    if (most > FIX_OWN) {
+        most -= FIX_OWN;
+        left -= min(left, FIX_OWN);
+        head += (size_t)RW * 2 * FIX_OWN;
+        constexpr uint32_t TREE = LANES == 4 ? 4 : 3;   // log2 GROUPS
+        uint32_t together = left ? (left + GROUPS - 1) / GROUPS + TREE + 1 : 0;
+        for (int m = 32; m >= LANES; m >>= 1) together += (uint32_t)__shfl_xor((int)together, m);
+        if (most <= together) {
+            add_own(most);
+        } else {
+            const uint32_t lane = threadIdx.x & 63, group = lane / LANES;
+            for (uint64_t m = __ballot(left > 0 && lane % LANES == 0); m; m &= m - 1) {
+                const int src = __ffsll((unsigned long long)m) - 1;
+                const uint32_t n = (uint32_t)__shfl((int)left, src);
+                const uint64_t p = (uint64_t)head;
+                const uint32_t* run = (const uint32_t*)((uint64_t)(uint32_t)__shfl((int)(uint32_t)p, src) |
+                                                        (uint64_t)(uint32_t)__shfl((int)(uint32_t)(p >> 32), src) << 32);
+                A x;
+                x.set_inf();
+                for (uint32_t i = 0; i < n; i += GROUPS) {
+                    A y;
+                    if (i + group < n) y = A::load_raw(run + (size_t)RW * 2 * (i + group));
+                    else y.set_inf();
+                    x.add(y);
+                }
+                for (int off = 32; off >= LANES; off >>= 1) x.add(x.from_lane((int)lane + off));   // group 0 has the sum
+                A y = x.from_lane((int)(lane % LANES));
+                if (group != (uint32_t)src / LANES) y.set_inf();
+                acc.add(y);
+            }
+        }
+    }
+    if (dst) acc.store_raw(dst);
 }
 
+// ------------------------------------------------------------------ 7. bucket reduction
 // log2 of the buckets of a part where a window has several, else 0
 __host__ __device__ inline uint32_t window_part_log(const MsmInst& d) {
     uint32_t k = 0;
@@ -442,7 +500,6 @@ __host__ __device__ inline uint32_t window_part_log(const MsmInst& d) {
     return k;
 }
 
-// ------------------------------------------------------------------ 7. bucket reduction
 // A window's value is sum_{d=1..NB} d * B_d. Workgroup per (window, part of
 // NB / S buckets), each lane group (slot) of it takes the g consecutive
 // buckets t*g .. t*g + g-1 of the part: with A_t = sum_q (q+1) B and R_t =
@@ -821,7 +878,9 @@ static void msm_device_stages(hzk_ctx* ctx, const MsmBatchLayout& L, char* base)
         for (uint32_t lv = 0; lv < L.hot_levels; ++lv, stride *= hot_seg<F>())
             hipLaunchKernelGGL(k_msm_hot_sum<F>, dim3(std::min<unsigned>(blocks_for(L.tot[SP_CHUNK], 256), 1024)), dim3(256), 0, st, b,
                                (const uint32_t*)sb.offs, (const uint32_t*)chunk2key, stride, (uint32_t*)carry);
-        hipLaunchKernelGGL(k_msm_fixup<F>, dim3(blocks_for(L.tot[SP_CHUNK] * LanePoint<F>::LANES, 256)), dim3(256), 0, st, b,
+        const bool by_key = L.tot[SP_KEY] < L.tot[SP_CHUNK];
+        hipLaunchKernelGGL((by_key ? k_msm_fixup<F, true> : k_msm_fixup<F, false>),
+                           dim3(blocks_for(std::min(L.tot[SP_KEY], L.tot[SP_CHUNK]) * LanePoint<F>::LANES, 256)), dim3(256), 0, st, b,
                            (const uint32_t*)sb.offs, (const uint32_t*)chunk2key, (const uint32_t*)carry, (uint32_t*)bucket);
     }
     {

@@ -85,3 +85,25 @@ def test_window_parts(ctx, orc, group, regime, n):
     finally:
         set_plan(group, log_n, 0)
         ctx.set_msm_regime(-1)
+
+
+# chunks a bucket continues into, where its fix-up changes hands: by itself, by the whole
+# wave (one long run among short ones), all runs long, more than 64 (summed beforehand);
+# groups numbered by chunk (many buckets) and by bucket (few)
+@pytest.mark.parametrize("group", [1, 2])
+@pytest.mark.parametrize("c", [4, 12])
+@pytest.mark.parametrize("runs", [[3, 1, 2], [4, 5, 4, 6], [60, 2, 2, 3, 2], [64], [65, 63, 1], [20] * 7, [130, 5, 64, 65, 9]])
+def test_fixup_runs(ctx, orc, group, c, runs):
+    digits = np.concatenate([np.full(K * r + 1, d + 1) for d, r in enumerate(runs)])
+    np.random.default_rng(3).shuffle(digits)
+    n = len(digits)
+    s = np.concatenate([pm.int_to_limbs(pm.to_mont(int(v), pm.R)) for v in digits])
+    k = orc.gen_fr(24, group, n)
+    bases = (orc.g1_mul_gen if group == 1 else orc.g2_mul_gen)(k)
+    log_n = n.bit_length() - 1
+    ctx.msm_tune_set(group, log_n, c, K, 1)
+    try:
+        got = _run(ctx, group, s, bases, n)
+    finally:
+        ctx.msm_tune_set(group, log_n, 0)
+    assert np.array_equal(got, orc.msm_closed_form(s, k, group))
