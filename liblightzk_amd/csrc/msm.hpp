@@ -19,6 +19,7 @@ struct MsmPlan {
     uint32_t NB;    // buckets per window, 2^(c-1)
     uint32_t K;     // sorted entries per accumulation lane (chunk length)
     uint32_t g;     // buckets per bucket-reduction run
+    bool fit = false;   // K is the built-in table's: msm_fit_chunks may move it
 };
 // Plan for n points: autotuned entry for the size class if one is loaded,
 // else the built-in heuristic; force_c / force_g override (0 = automatic).

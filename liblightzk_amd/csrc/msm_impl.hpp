@@ -3,6 +3,7 @@
 // translation unit. Stages 1-4 and the batch layout are described in msm.hip.
 #pragma once
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <map>
 #include <vector>
@@ -683,8 +684,47 @@ struct MsmBatchLayout {
     size_t o_upload_end = 0, o_download_end = 0;
 };
 
+// Chunk lengths between 3/4 and 2 times the plans' that give the SIMDs equal
+// work. The accumulation issues one wave's instructions at a time on a SIMD,
+// so it takes K additions times the waves of the fullest SIMD (a wave alone
+// issues 1.2 times slower), and a chunk more costs the fix-up about 4.5
+// additions of a wave per 64. The plans are tuned at one size of a class of
+// [2^k, 2^(k+1)); at others a last, nearly empty round cost up to a third:
+// G2 65536 points 806 -> 745 us, 131072 1077 -> 996; G1 50000 399 -> 382, 420000
+// 1031 -> 949; 32 G1 MSMs of a batch 3300 -> 2910. How many digits
+// are zero is known on the GPU only: the cost is that of all and of the third
+// that a witness of 0/1 flags leaves (2^20 witness by the first alone: 1133 ->
+// 1252). Above 16 waves a SIMD it gains less than the model knows.
+static constexpr double MSM_SPARSE = 0.32;
+static void msm_fit_chunks(const hzk_ctx* ctx, MsmInst* inst, const uint8_t* fit, size_t count) {
+    const auto scaled = [&](size_t i, uint32_t q) {
+        return fit[i] ? (inst[i].K * q / 16 + 3) & ~3u : inst[i].K;   // a multiple of 4, as the plans are
+    };
+    const auto cost = [&](uint32_t q, double share) {   // share: digits that are not zero
+        uint64_t entries = 0, chunks = 0;
+        for (size_t i = 0; i < count; ++i) {
+            const uint64_t e = (uint64_t)inst[i].n * inst[i].W, K = scaled(i, q);
+            entries += e;
+            chunks += (e + K - 1) / K;
+        }
+        const double waves = share * (double)((chunks + 255) / 256) / ctx->num_cus;   // per SIMD
+        return (double)entries / chunks * (waves <= 1 ? 1.2 : std::ceil(waves)) + 4.5 * waves;
+    };
+    uint64_t chunks = 0;
+    for (size_t i = 0; i < count; ++i) chunks += (uint64_t)inst[i].n * inst[i].W / inst[i].K;
+    if (chunks > (uint64_t)ctx->num_cus * 256 * 16) return;
+    uint32_t best = 16;
+    double least = 0.97 * (cost(16, 1) + cost(16, MSM_SPARSE));
+    for (uint32_t q = 12; q <= 32; ++q) {
+        const double c = cost(q, 1) + cost(q, MSM_SPARSE);
+        if (c < least) least = c, best = q;
+    }
+    for (size_t i = 0; i < count; ++i) inst[i].K = scaled(i, best);
+}
+
+// longer: chunks of that many times the plans' length (less scratch)
 template <class F>
-static MsmBatchLayout msm_layout(hzk_ctx* ctx, const MsmJob* jobs, size_t count) {
+static MsmBatchLayout msm_layout(hzk_ctx* ctx, const MsmJob* jobs, size_t count, uint32_t longer = 1) {
     MsmBatchLayout L;
     L.inst.resize(count);
     L.begin.assign((size_t)SP_COUNT * (count + 1), 0);
@@ -702,6 +742,7 @@ static MsmBatchLayout msm_layout(hzk_ctx* ctx, const MsmJob* jobs, size_t count)
         regime = msm_wide_batch(g2, count, e) ? MSM_REGIME_BATCH : MSM_REGIME_SINGLE;
     }
     L.regime = regime;
+    std::vector<uint8_t> fit(count);
     for (size_t i = 0; i < count; ++i) {
         MsmPlan p = msm_plan_ctx(ctx, g2, jobs[i].n, (int)jobs[i].win_siz, regime);
         MsmInst& d = L.inst[i];
@@ -735,6 +776,12 @@ static MsmBatchLayout msm_layout(hzk_ctx* ctx, const MsmJob* jobs, size_t count)
             while (K < 4096 && entries / (2 * (uint64_t)K) >= ((uint64_t)1 << 18)) K <<= 1;
             d.K = K;
         }
+        fit[i] = p.fit && jobs[i].levels <= 1;
+        d.K *= longer;
+    }
+    if (longer == 1) msm_fit_chunks(ctx, L.inst.data(), fit.data(), count);
+    for (size_t i = 0; i < count; ++i) {
+        MsmInst& d = L.inst[i];
         // parts per window: one run of g buckets per slot of a window-sum
         // workgroup, at most 64 parts (host combine, lanes of the device combine)
         const uint32_t slots = regime == MSM_REGIME_BATCH ? LdsLanes<F, 64>::SLOTS : LdsLanes<F, 256>::SLOTS;
@@ -948,7 +995,8 @@ int msm_batch_run(hzk_ctx* ctx, const MsmJob* jobs, size_t count, int dests_on_h
         HZK_CHECK(ctx, (uint64_t)L.inst[i].n * L.inst[i].W <= 0xffff0000ull, HZK_ERR_UNSUPPORTED,
                   "msm: n=%u with %u windows exceeds 2^32 bucket entries", L.inst[i].n, L.inst[i].W);
     int rc = 0;
-    if (ext_scratch) {
+    if (ext_scratch) {   // longer chunks need less
+        for (uint32_t longer = 2; L.bytes > ext_bytes && longer <= 4; longer *= 2) L = msm_layout<F>(ctx, jobs, count, longer);
         HZK_CHECK(ctx, L.bytes <= ext_bytes && !capture, HZK_ERR_UNSUPPORTED,
                   "msm: this MSM needs %zu bytes of scratch, the static buffer holds %zu", L.bytes, ext_bytes);
     } else {
