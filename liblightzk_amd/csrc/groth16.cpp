@@ -475,7 +475,8 @@ static size_t msm_scratch_bound(size_t n, size_t pt_bytes) {
     const size_t raw = pt_bytes / 8 * 9;
     size_t worst = 0;
     for (int regime : {MSM_REGIME_SINGLE, MSM_REGIME_BATCH}) {
-        const MsmPlan p = msm_plan_builtin(pt_bytes > 128, n, regime);
+        MsmPlan p = msm_plan_builtin(pt_bytes > 128, n, regime);
+        msm_widen(pt_bytes > 128, n, p);
         const size_t W = p.W, nk = W * p.NB, entries = n * W, chunks = entries * 4 / (3 * p.K) + 1;   // K may shrink by a quarter
         const size_t cg = msm_coarse_groups(n, p.NB, p.W), groups = W * cg, pieces = entries / MSM_SUB + groups;
         size_t b = entries * 14 + groups * msm_tiles(n) * 4 + pieces * (p.NB / cg) * 4 + (nk + 1) * 4 + (nk + 1) * raw +

@@ -745,6 +745,7 @@ static MsmBatchLayout msm_layout(hzk_ctx* ctx, const MsmJob* jobs, size_t count,
     std::vector<uint8_t> fit(count);
     for (size_t i = 0; i < count; ++i) {
         MsmPlan p = msm_plan_ctx(ctx, g2, jobs[i].n, (int)jobs[i].win_siz, regime);
+        if (p.fit) msm_widen(g2, jobs[i].n, p);
         MsmInst& d = L.inst[i];
         d.scalars = jobs[i].scalars;
         d.bases = jobs[i].bases;

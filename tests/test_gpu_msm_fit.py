@@ -23,6 +23,16 @@ def test_sizes(ctx, orc, group, n):
     assert np.array_equal(out.download(np.uint64, 12 * group), want)
 
 
+def test_wide_windows(ctx, orc):
+    """17-bit windows of the largest G1 MSMs, digits of every sign and size."""
+    n = (1 << 22) + 5
+    ds, db, want = _inputs(ctx, orc, 1, 33, n)
+    out = ctx.alloc(96)
+    ctx.msm_g1(ds, db, n, out)
+    assert ctx.msm_last_stats()["c"] == 17
+    assert np.array_equal(out.download(np.uint64, 12), want)
+
+
 @pytest.mark.parametrize("graph", [False, True])
 def test_instances(ctx, orc, graph):
     sizes = [1, 300, 4097, 60000, 110003, 33000]
