@@ -23,7 +23,7 @@ def _run(ctx, group, s, bases, n):
     return dd.download(np.uint64, 12 * group)
 
 
-# chunks of the bucket beyond its first: 16 is fixed up serially; a segment is 1024 (G1) or 512 (G2) chunks
+# chunks of the bucket beyond its first: up to 64 are fixed up; beyond, a segment is 1024 (G1) or 512 (G2) chunks
 @pytest.mark.parametrize("group", [1, 2])
 @pytest.mark.parametrize("chunks", [1, 2, 16, 17, 18, 512, 513, 514, 1025, 1026, 2100])
 @pytest.mark.parametrize("points", ["equal", "distinct", "opposite"])
