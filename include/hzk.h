@@ -163,8 +163,8 @@ int hzk_pointwise_abc(hzk_ctx* ctx, size_t deg, void* A, const void* B, const vo
  * hzk_msm_g1 with base_layout HZK_BASES_AFFINE and win_siz 0 (dest: device
  * pointer to 96 bytes). Its scratch is a static device array of
  * HZK_NOALLOC_SCRATCH_MB MiB per GPU (mapped when a context is created, held
- * until the process ends); an MSM whose plan needs more (about n > 2^15
- * points) fails with HZK_ERR_UNSUPPORTED. All calls on one GPU share that
+ * until the process ends); an MSM whose plan needs more even with chunks 4
+ * times as long (about n > 330000 points) fails with HZK_ERR_UNSUPPORTED. All calls on one GPU share that
  * array: calls that overlap on one GPU, from any contexts, race. Host
  * bookkeeping uses the C++ heap and pageable copies; nothing is allocated on
  * the device or pinned. */
