@@ -144,4 +144,40 @@ struct fr29 {
     }
 };
 
+// ---- signed limbs (V: nine int32_t limbs l, limb29.hpp's)
+// A value in (-300 r, 600 r), limbs within +-2^31, brought into [0, 2r): q r
+// subtracted with q = floor((l8 - 4 + 320 r8) / (r8 + 1)) - 320, at most the
+// true quotient (limbs 0..7 may borrow up to 4 from limb 8). The dividend stays
+// in [0, 2^32): 920 r8 < 2^31.5.
+template <class V>
+HZK_DEV V fr_reduce(const V& v) {
+    constexpr uint32_t r8 = fr29::P[8];
+    const int32_t q = (int32_t)(((uint32_t)v.l[8] + (320 * r8 - 4)) / (r8 + 1)) - 320;
+    V r;
+    int64_t c = 0;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+        c += (int64_t)v.l[i] - (int64_t)q * (int32_t)fr29::P[i];
+        r.l[i] = (int32_t)((uint32_t)c & fr29::MASK);
+        c >>= 29;
+    }
+    return r;
+}
+// [0, 2r) -> [0, r)
+template <class V>
+HZK_DEV V fr_canonical(const V& v) {
+    V d;
+    int32_t c = 0;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+        const int32_t t = v.l[i] - (int32_t)fr29::P[i] + c;
+        d.l[i] = t & (int32_t)fr29::MASK;
+        c = t >> 29;
+    }
+    V r;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) r.l[i] = c < 0 ? v.l[i] : d.l[i];
+    return r;
+}
+
 }  // namespace hzk

@@ -96,37 +96,6 @@ HZK_DEV fr_t fr_pack(const limbs29& v) {
     x.l[0] = a.x, x.l[1] = a.y, x.l[2] = a.z, x.l[3] = a.w, x.l[4] = b.x, x.l[5] = b.y, x.l[6] = b.z, x.l[7] = b.w;
     return x;
 }
-// a value in (-48 r, 600 r), limbs within +-2^31, brought into [0, 2r): q r
-// subtracted with q = floor((l8 - 4 + 64 r8) / (r8 + 1)) - 64, at most the true
-// quotient (limbs 0..7 may borrow up to 4 from limb 8)
-HZK_DEV limbs29 fr_reduce(const limbs29& v) {
-    constexpr uint32_t r8 = Fr29Mod::P[8];
-    const int32_t q = (int32_t)(((uint32_t)v.l[8] + (64 * r8 - 4)) / (r8 + 1)) - 64;
-    limbs29 r;
-    int64_t c = 0;
-#pragma unroll
-    for (int i = 0; i < 9; ++i) {
-        c += (int64_t)v.l[i] - (int64_t)q * (int32_t)Fr29Mod::P[i];
-        r.l[i] = (int32_t)((uint32_t)c & MASK29);
-        c >>= 29;
-    }
-    return r;
-}
-// [0, 2r) -> [0, r)
-HZK_DEV limbs29 fr_canonical(const limbs29& v) {
-    limbs29 d;
-    int32_t c = 0;
-#pragma unroll
-    for (int i = 0; i < 9; ++i) {
-        const int32_t t = v.l[i] - (int32_t)Fr29Mod::P[i] + c;
-        d.l[i] = t & (int32_t)MASK29;
-        c = t >> 29;
-    }
-    limbs29 r;
-#pragma unroll
-    for (int i = 0; i < 9; ++i) r.l[i] = c < 0 ? v.l[i] : d.l[i];
-    return r;
-}
 // 32 x, reduced: a 2^256-form factor made a 2^261-form one
 HZK_DEV limbs29 fr_times32(const limbs29& x) {
     limbs29 r;
@@ -326,10 +295,13 @@ HZK_DEV void ntt_store(limbs29* v, const NttPassDesc& d, const NttTile& T, uint3
 // the chunk's stage bits; its other tile bits come from the thread index (low
 // bits first, so a wave's lanes read consecutive elements wherever L > 0). A
 // chunk's twiddles are loaded before the exchange that leads to it.
-// Bounds, in units of r: an element enters below 2. DIF sums double, so
-// after at most 8 stages they stay below 512 (products come back below 5);
-// a pass of more stages reduces every element after the sixth. DIT elements
-// grow by less than 1.7 a stage.
+// Bounds, in units of r: an element enters in [0, 2). DIF sums double in both
+// directions; a product of a difference (-2^(s+1), 2^(s+1)) after s stages lies
+// above -2^(s+1)/169 (twice that with a caller's table), so after eight stages
+// sums stay in (-4, 512). The last two stages over the library's tables leave
+// differences unmultiplied: after six stages sums of two are in (-2, 256), their
+// differences in (-258, 258). A pass of more than eight stages reduces every
+// element after the sixth. DIT elements grow by less than 1.7 a stage.
 template <bool DIT, int TB>
 HZK_DEV void ntt_tile(const NttPassDesc& d, uint32_t b, uint4* sh) {
     constexpr int LE = 2, E = 4;
