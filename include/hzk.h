@@ -125,7 +125,12 @@ int hzk_msm_last_stats(hzk_ctx* ctx, uint32_t* out5);
  * omega_powers: device table w^e for e < deg/2 (ntt_setup layout,
  * include/protocol/groth16-operator.cuh:6-32), or NULL for the library's own
  * table of the primitive deg-th root (inverse = 0) or its inverse (inverse = 1,
- * then scaled by 1/deg unless factor is given). factor: device Fr or NULL. */
+ * then scaled by 1/deg unless factor is given). factor: device Fr or NULL.
+ * From about 2^10 points on, transforms of natural order (single and batched)
+ * use a workspace as large as the call's data (2 GiB at 2^26), which the context
+ * keeps for the next one. It gives it back when one of its own allocations finds
+ * the device full, and without room for it the transform runs in place,
+ * slower. */
 int hzk_ntt(hzk_ctx* ctx, void* coeffs, size_t deg, const void* omega_powers, int inverse, const void* factor);
 /* The reference's ntt_setup table for an M-point domain, written to host
  * memory as 6M + 2 Fr elements (replaces ntt_setup<FieldT, ntt_config*>,
@@ -341,7 +346,9 @@ int hzk_msm_batch_autotune(hzk_ctx* ctx, int group, int log_min, int log_max, do
 int hzk_set_tuning(hzk_ctx* ctx, int window_bits, int segment);
 /* MSM plan regime: -1 by batch width (default), 0 single-MSM plans, 1 wide-batch plans */
 int hzk_set_msm_regime(hzk_ctx* ctx, int regime);
-/* make the n-th following scratch allocation fail with HZK_ERR_NOMEM (-1 = off) */
+/* make the n-th following scratch allocation fail with HZK_ERR_NOMEM (-1 = off;
+ * -2: the next allocation finds the device full until the context has given
+ * back the memory it keeps for speed alone) */
 int hzk_inject_alloc_failure(hzk_ctx* ctx, long after_n);
 
 #ifdef __cplusplus

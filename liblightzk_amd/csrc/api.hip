@@ -21,6 +21,31 @@ int set_error(hzk_ctx* ctx, int code, const char* fmt, ...) {
     return code;
 }
 
+// test hook: the device is full until give_back
+static bool alloc_fails(const hzk_ctx* ctx) { return ctx->fail_alloc_after == -2; }
+
+bool give_back(hzk_ctx* ctx) {
+    if (alloc_fails(ctx)) ctx->fail_alloc_after = -1;
+    if (!ctx->ntt_ws) return false;
+    (void)hipFreeAsync(ctx->ntt_ws, ctx->stream);
+    ctx->ntt_ws = nullptr;
+    ctx->ntt_ws_bytes = 0;
+    (void)hipStreamSynchronize(ctx->stream);
+    hipMemPool_t pool;   // freed memory would stay cached there
+    if (hipDeviceGetDefaultMemPool(&pool, ctx->device) == hipSuccess) (void)hipMemPoolTrimTo(pool, 0);
+    (void)hipGetLastError();
+    return true;
+}
+
+hipError_t device_malloc(hzk_ctx* ctx, void** out, size_t bytes) {
+    hipError_t e = alloc_fails(ctx) ? hipErrorOutOfMemory : hipMalloc(out, bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        if (give_back(ctx)) e = hipMalloc(out, bytes);
+    }
+    return e;
+}
+
 int ensure_scratch(hzk_ctx* ctx, size_t bytes) {
     if (ctx->fail_alloc_after >= 0) {
         if (ctx->fail_alloc_after == 0) {
@@ -43,11 +68,15 @@ int ensure_scratch(hzk_ctx* ctx, size_t bytes) {
         ctx->scratch_bytes = 0;
     }
     size_t want = std::max(bytes + bytes / 8, 2 * old);
-    hipError_t e = hipMallocAsync(&ctx->scratch, want, ctx->stream);
+    hipError_t e = alloc_fails(ctx) ? hipErrorOutOfMemory : hipMallocAsync(&ctx->scratch, want, ctx->stream);
     if (e != hipSuccess) {
         (void)hipGetLastError();
-        e = hipMallocAsync(&ctx->scratch, bytes, ctx->stream);
         want = bytes;
+        e = alloc_fails(ctx) ? hipErrorOutOfMemory : hipMallocAsync(&ctx->scratch, want, ctx->stream);
+    }
+    if (e != hipSuccess && give_back(ctx)) {
+        (void)hipGetLastError();
+        e = hipMallocAsync(&ctx->scratch, want, ctx->stream);
     }
     if (e != hipSuccess) {
         (void)hipGetLastError();
@@ -282,7 +311,7 @@ int hzk_device_sync(hzk_ctx* ctx) {
 
 int hzk_device_alloc(hzk_ctx* ctx, size_t bytes, void** out) {
     if (!ctx || !out) return HZK_ERR_INVALID;
-    hipError_t e = hipMalloc(out, bytes ? bytes : 1);
+    hipError_t e = device_malloc(ctx, out, bytes ? bytes : 1);
     if (e != hipSuccess) {
         (void)hipGetLastError();
         *out = nullptr;

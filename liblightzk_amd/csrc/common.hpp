@@ -49,7 +49,8 @@ struct hzk_ctx {
     std::vector<Rec> pending;
     std::map<std::string, std::pair<double, long>> totals;   // name -> (ms, launches)
     std::vector<hipEvent_t> event_pool;
-    // fault injection for tests of the error paths (host-side only)
+    // fault injection for tests of the error paths (host-side only); -2: the
+    // next allocation finds the device full until a workspace is given back
     long fail_alloc_after = -1;
     // fixed-base comb tables (device, built on first use)
     void* comb_g1 = nullptr;
@@ -62,7 +63,7 @@ struct hzk_ctx {
     // NTT twiddle / coset tables for the last transform size (ntt.hip)
     void* ntt_cache = nullptr;
     // workspace of transforms that permute on their last pass (ntt.hip): grown
-    // on demand in stream order, freed at destroy
+    // on demand in stream order, freed at destroy or when an allocation fails
     void* ntt_ws = nullptr;
     size_t ntt_ws_bytes = 0;
     // MSM plans [regime][G1, G2][log2 n]; regime 0: an MSM that has the GPU
@@ -115,6 +116,11 @@ void timing_merge(hzk_ctx* ctx, hzk_ctx* from);
 int stage_acquire(hzk_ctx* ctx, size_t bytes, char** buf, int* slot);
 int stage_fence(hzk_ctx* ctx, int slot);
 void ntt_release(hzk_ctx* ctx);
+// Device memory that the context keeps for speed alone (the transforms'
+// workspace) back to the device; false when there was none.
+bool give_back(hzk_ctx* ctx);
+// hipMalloc, tried again once the context has given back what it can
+hipError_t device_malloc(hzk_ctx* ctx, void** out, size_t bytes);
 int spmv3(hzk_ctx* ctx, const hzk_csr* A, const hzk_csr* B, const hzk_csr* C, const void* z, void* Az, void* Bz, void* Cz);
 int pointwise_abc(hzk_ctx* ctx, size_t n, void* A, const void* B, const void* C, const void* scale);
 // dst[k] = src[idx[k]], k < n, for elements of elem_bytes (a multiple of 16) on ctx's stream

@@ -150,7 +150,7 @@ Fr row_dot(const HostCsr& m, size_t rows, size_t r, const Fr* z) {
 template <class T>
 int dev_upload(hzk_ctx* ctx, hzk_g16* g, const T* src, size_t bytes, void** out) {
     void* d = nullptr;
-    HZK_HIP(ctx, hipMalloc(&d, bytes ? bytes : 1));
+    HZK_HIP(ctx, device_malloc(ctx, &d, bytes ? bytes : 1));
     g->own(d, bytes);
     if (bytes) HZK_HIP(ctx, hipMemcpy(d, src, bytes, hipMemcpyHostToDevice));
     *out = d;
@@ -159,7 +159,7 @@ int dev_upload(hzk_ctx* ctx, hzk_g16* g, const T* src, size_t bytes, void** out)
 
 int dev_alloc(hzk_ctx* ctx, hzk_g16* g, size_t bytes, void** out) {
     void* d = nullptr;
-    HZK_HIP(ctx, hipMalloc(&d, bytes ? bytes : 1));
+    HZK_HIP(ctx, device_malloc(ctx, &d, bytes ? bytes : 1));
     g->own(d, bytes);
     *out = d;
     return 0;
@@ -173,7 +173,7 @@ int key_points(hzk_ctx* ctx, hzk_g16* g, const std::vector<Fr>& k, void** out) {
     if (rc) return rc;
     if (n == 0) return 0;
     void* ds = nullptr;
-    HZK_HIP(ctx, hipMalloc(&ds, n * 32));
+    HZK_HIP(ctx, device_malloc(ctx, &ds, n * 32));
     HZK_HIP(ctx, hipMemcpy(ds, k.data(), n * 32, hipMemcpyHostToDevice));
     rc = G2 ? hzk_fixbase_g2(ctx, ds, n, *out) : hzk_fixbase_g1(ctx, ds, n, *out);
     (void)hipStreamSynchronize(ctx->stream);

@@ -36,7 +36,7 @@ int put_device(hzk_ctx* ctx, Writer& w, const void* dev, size_t bytes, std::vect
 // file -> new device array (owned by g)
 int get_device(hzk_ctx* ctx, Reader& r, hzk_g16* g, size_t bytes, void** out, std::vector<char>& stage) {
     void* d = nullptr;
-    HZK_HIP(ctx, hipMalloc(&d, bytes ? bytes : 1));
+    HZK_HIP(ctx, device_malloc(ctx, &d, bytes ? bytes : 1));
     g->own(d, bytes);
     *out = d;
     for (size_t off = 0; off < bytes && r.ok; off += STAGE) {
@@ -156,7 +156,7 @@ int hzk_g16_load(hzk_ctx* ctx, const char* path, hzk_g16** out) {
                 {m.val.data(), m.val.size() * 32}, {m.col.data(), m.col.size() * 8}, {m.row_ptr.data(), m.row_ptr.size() * 8}};
             void** dst[3] = {&g->d_val[i], (void**)&g->d_col[i], (void**)&g->d_rp[i]};
             for (int k = 0; k < 3 && !rc; ++k) {
-                hipError_t e = hipMalloc(&d, parts[k].second ? parts[k].second : 1);
+                hipError_t e = device_malloc(ctx, &d, parts[k].second ? parts[k].second : 1);
                 if (e == hipSuccess) {
                     g->own(d, parts[k].second);
                     *dst[k] = d;

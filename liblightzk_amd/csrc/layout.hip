@@ -123,7 +123,7 @@ int ref_bases_affine(hzk_ctx* ctx, int group, const void* ref, size_t n, const v
             ctx->conv = nullptr;
             ctx->conv_bytes = 0;
         }
-        hipError_t e = hipMalloc(&ctx->conv, bytes);
+        hipError_t e = device_malloc(ctx, &ctx->conv, bytes);
         if (e != hipSuccess) {
             (void)hipGetLastError();
             return set_error(ctx, HZK_ERR_NOMEM, "conversion buffer of %zu bytes: %s", bytes, hipGetErrorString(e));

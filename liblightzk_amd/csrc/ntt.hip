@@ -631,8 +631,8 @@ static int ensure_tables(hzk_ctx* ctx, int logn, NttTables** out) {
     host::Fr ninv = fr_from_u64(n).inverse();
     const host::Fr to261 = fr_from_u64(32);
     for (int d = 0; d < 2; ++d) {
-        HZK_HIP(ctx, hipMalloc(&t.tw[d], half * 32));
-        HZK_HIP(ctx, hipMalloc(&t.coset[d], n * 32));
+        HZK_HIP(ctx, device_malloc(ctx, (void**)&t.tw[d], half * 32));
+        HZK_HIP(ctx, device_malloc(ctx, (void**)&t.coset[d], n * 32));
         int rc = fill_powers(ctx, t.tw[d], half, d ? wi : w, to261);
         if (rc) return rc;
         rc = fill_powers(ctx, t.coset[d], n, d ? gi : g, d ? to261 * ninv : to261);
@@ -649,7 +649,7 @@ static int ensure_rev_tables(hzk_ctx* ctx, int logn, NttTables* t) {
     if (t->coset_rev[0]) return 0;
     const size_t n = (size_t)1 << logn;
     for (int d = 0; d < 2; ++d) {
-        HZK_HIP(ctx, hipMalloc(&t->coset_rev[d], n * 32));
+        HZK_HIP(ctx, device_malloc(ctx, (void**)&t->coset_rev[d], n * 32));
         hipLaunchKernelGGL(k_bitrev_table, dim3(blocks_for(n, 256)), dim3(256), 0, ctx->stream, t->coset_rev[d],
                            (const fr_t*)t->coset[d], logn, d ? (const fr_t*)nullptr : (const fr_t*)t->ninv);
         HZK_HIP(ctx, hipGetLastError());
@@ -752,16 +752,19 @@ static fr_t* ntt_workspace(hzk_ctx* ctx, uint64_t elems) {
     if (hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return nullptr;
     const size_t bytes = (size_t)elems * 32;
     if (ctx->ntt_ws_bytes >= bytes) return (fr_t*)ctx->ntt_ws;
+    const size_t doubled = 2 * ctx->ntt_ws_bytes;   // slowly growing calls settle after a few steps
     if (ctx->ntt_ws) (void)hipFreeAsync(ctx->ntt_ws, ctx->stream);
     ctx->ntt_ws = nullptr;
     ctx->ntt_ws_bytes = 0;
-    if (hipMallocAsync(&ctx->ntt_ws, bytes, ctx->stream) != hipSuccess) {
+    for (const size_t want : {std::max(bytes, doubled), bytes}) {
+        if (hipMallocAsync(&ctx->ntt_ws, want, ctx->stream) == hipSuccess) {
+            ctx->ntt_ws_bytes = want;
+            return (fr_t*)ctx->ntt_ws;
+        }
         (void)hipGetLastError();
         ctx->ntt_ws = nullptr;
-        return nullptr;
     }
-    ctx->ntt_ws_bytes = bytes;
-    return (fr_t*)ctx->ntt_ws;
+    return nullptr;
 }
 
 static uint64_t pass_tiles(const NttPassDesc& d) { return (uint64_t)1 << (d.k - d.R - d.gl - d.hb); }
