@@ -325,10 +325,15 @@ int hzk_roofline_probe(hzk_ctx* ctx, int kind, double* value);
  * do not depend on the plan. c = 0 clears the entry (built-in table or
  * heuristic). */
 int hzk_msm_tune_set(hzk_ctx* ctx, int group, int log_n, int c, uint32_t K, uint32_t g);
-/* the plan an MSM of 2^log_n points would use now */
+/* the same for a plan that hzk_msm_autotune (batch = 0) or
+ * hzk_msm_batch_autotune (batch = 1) found: like the built-in ones it is fitted
+ * to each MSM's size (K by a factor of 3/4 to 2; 17-bit windows for c = 16 from
+ * 2^22 G1 points on), while a plan given to hzk_msm_tune_set runs as it is */
+int hzk_msm_tune_load(hzk_ctx* ctx, int batch, int group, int log_n, int c, uint32_t K, uint32_t g);
+/* the plan of an MSM of 2^log_n points, before it is fitted to the size */
 int hzk_msm_tune_get(hzk_ctx* ctx, int group, int log_n, int* c, uint32_t* K, uint32_t* g);
 /* time candidate plans for classes log_min..log_max on seeded synthetic
- * inputs (coordinate descent over c, K, g; at most budget_ms per class) and
+ * inputs of 1.2 * 2^log_n points (coordinate descent over c, K, g; at most budget_ms per class) and
  * store the fastest in the context's table */
 int hzk_msm_autotune(hzk_ctx* ctx, int group, int log_min, int log_max, double budget_ms);
 /* The same for the throughput regime: the plans used by the instances of a
@@ -336,7 +341,7 @@ int hzk_msm_autotune(hzk_ctx* ctx, int group, int log_min, int log_max, double b
  * reaches 2^26, or at least 8 G1 / 16 G2 MSMs with 2^24 digits), which fills
  * the GPU without help from the plan; typically
  * fewer window bits (fewer buckets to reduce), longer chunks and runs. The
- * autotuner times each class as a batch of 2^26 / (16 n) instances (2..256). */
+ * autotuner times each class as a batch of 2^26 / (16 * 2^log_n) instances (2..256). */
 int hzk_msm_batch_tune_set(hzk_ctx* ctx, int group, int log_n, int c, uint32_t K, uint32_t g);
 int hzk_msm_batch_tune_get(hzk_ctx* ctx, int group, int log_n, int* c, uint32_t* K, uint32_t* g);
 int hzk_msm_batch_autotune(hzk_ctx* ctx, int group, int log_min, int log_max, double budget_ms);

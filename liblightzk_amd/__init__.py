@@ -181,6 +181,10 @@ class Context:
     def msm_tune_set(self, group, log_n, c, K=0, g=0):
         self._check(load().hzk_msm_tune_set(self.handle, group, log_n, c, K, g))
 
+    def msm_tune_load(self, group, log_n, c, K, g, batch=False):
+        """A plan that the autotuner found: fitted to each MSM's size like the built-in ones."""
+        self._check(load().hzk_msm_tune_load(self.handle, 1 if batch else 0, group, log_n, c, K, g))
+
     def msm_tune_get(self, group, log_n):
         c, K, g = ctypes.c_int(), ctypes.c_uint32(), ctypes.c_uint32()
         self._check(load().hzk_msm_tune_get(self.handle, group, log_n, ctypes.byref(c), ctypes.byref(K), ctypes.byref(g)))

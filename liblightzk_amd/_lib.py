@@ -100,6 +100,7 @@ def load():
         "hzk_set_tuning": (i32, [vp, i32, i32]),
         "hzk_set_msm_regime": (i32, [vp, i32]),
         "hzk_msm_tune_set": (i32, [vp, i32, i32, i32, u32, u32]),
+        "hzk_msm_tune_load": (i32, [vp, i32, i32, i32, i32, u32, u32]),
         "hzk_msm_tune_get": (i32, [vp, i32, i32, ctypes.POINTER(i32), ctypes.POINTER(u32), ctypes.POINTER(u32)]),
         "hzk_msm_autotune": (i32, [vp, i32, i32, i32, dbl]),
         "hzk_msm_batch_tune_set": (i32, [vp, i32, i32, i32, u32, u32]),

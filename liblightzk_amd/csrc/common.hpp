@@ -18,6 +18,7 @@ struct hzk_tune_entry {
     int c = 0;
     uint32_t K = 0;
     uint32_t g = 0;
+    bool fit = false;   // tuned, not a caller's: K and c may be fitted to the size (MsmPlan::fit)
 };
 
 struct hzk_ctx {

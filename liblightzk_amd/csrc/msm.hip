@@ -678,10 +678,12 @@ MsmPlan msm_plan_ctx(hzk_ctx* ctx, int g2, size_t n, int force_c, int regime) {
         const int cls = size_class(n), gi = g2 ? 1 : 0;
         for (int r = regime; r >= MSM_REGIME_SINGLE; --r) {
             hzk_tune_entry t = ctx->tune[r][gi][cls];
-            const bool builtin = !t.c && !ctx->force_seg;
-            if (builtin) t = BUILTIN_PLANS[r][gi][cls];
+            if (!t.c && !ctx->force_seg) {
+                t = BUILTIN_PLANS[r][gi][cls];
+                t.fit = true;
+            }
             if (plan_from_entry(t, n, ctx->force_seg, &p)) {
-                p.fit = builtin;
+                p.fit = t.fit;
                 break;
             }
         }

@@ -19,9 +19,9 @@ struct MsmPlan {
     uint32_t NB;    // buckets per window, 2^(c-1)
     uint32_t K;     // sorted entries per accumulation lane (chunk length)
     uint32_t g;     // buckets per bucket-reduction run
-    bool fit = false;   // K is the built-in table's: msm_fit_chunks may move it
+    bool fit = false;   // a tuned plan (built in, autotuned or loaded): msm_fit_chunks may move K, msm_widen c
 };
-// Built-in plans from MSM_WIDE_N G1 points on take 17-bit windows, one more
+// Tuned plans (size classes up to 2^24) from MSM_WIDE_N G1 points on take 17-bit windows, one more
 // than a caller may ask for: 15 of them instead of 16 save that part of the
 // accumulation and the sort, for twice the buckets: 2^23 points 10.89 -> 10.45
 // ms, 2^24 20.83 -> 20.14, 7 million 9.11 -> 8.89; 2^22 and less gain under 1 %.

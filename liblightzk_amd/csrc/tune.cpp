@@ -15,7 +15,9 @@
 // {K/4 .. 4K}, then g over powers of two (up to 32, or 64 in the batch
 // regime). Each candidate is the best of several timed runs after one
 // warm-up, on seeded uniform scalars and bases k_i * G generated on the
-// device. The winner is written to the context's table of that regime.
+// device, at 1.2 * 2^log_n points: inside its class rather than at the lower
+// end, with the chunk lengths and window bits that tuned plans are fitted to.
+// The winner is written to the context's table of that regime.
 #include <algorithm>
 #include <chrono>
 #include <cstring>
@@ -52,7 +54,7 @@ double time_msm(hzk_ctx* ctx, int group, const void* s, const void* b, size_t n,
     return best;
 }
 
-int tune_set(hzk_ctx* ctx, int regime, int group, int log_n, int c, uint32_t K, uint32_t g) {
+int tune_set(hzk_ctx* ctx, int regime, int group, int log_n, int c, uint32_t K, uint32_t g, bool fit = false) {
     if (!ctx) return HZK_ERR_INVALID;
     HZK_CHECK(ctx, (group == 1 || group == 2) && log_n >= 0 && log_n < 32, HZK_ERR_INVALID, "tune_set: group %d log_n %d",
               group, log_n);
@@ -64,6 +66,7 @@ int tune_set(hzk_ctx* ctx, int regime, int group, int log_n, int c, uint32_t K, 
     t.c = c;
     t.K = c ? K : 0;
     t.g = c ? g : 0;
+    t.fit = fit;
     return HZK_OK;
 }
 
@@ -78,6 +81,8 @@ int tune_get(hzk_ctx* ctx, int regime, int group, int log_n, int* c, uint32_t* K
     return HZK_OK;
 }
 
+size_t tune_points(int log_n) { return ((size_t)1 << log_n) + ((size_t)1 << log_n) / 5; }
+
 // Batch regime: a class is timed as a batch of B = 2^26 / (16 n) instances
 // (2 to 256), about the width at which a batch takes the throughput plans.
 uint32_t tune_batch_width(int log_n) {
@@ -89,13 +94,13 @@ int autotune(hzk_ctx* ctx, int regime, int group, int log_min, int log_max, doub
     if (!ctx) return HZK_ERR_INVALID;
     HZK_CHECK(ctx, (group == 1 || group == 2) && log_min >= 1 && log_min <= log_max && log_max <= 26, HZK_ERR_INVALID,
               "autotune: group %d, classes %d..%d", group, log_min, log_max);
-    const size_t nmax = (size_t)1 << log_max;
+    const size_t nmax = tune_points(log_max);
     const size_t pt = group == 1 ? 64 : 128;
     // scalars: the batch regime offsets instance i by i*step scalars
     size_t smax = nmax;
     if (regime == MSM_REGIME_BATCH)
         for (int L = log_min; L <= log_max; ++L) {
-            const size_t n = (size_t)1 << L, step = n / 64 + 1;
+            const size_t n = tune_points(L), step = n / 64 + 1;
             smax = std::max(smax, n + step * (tune_batch_width(L) - 1));
         }
     const uint32_t maxb = regime == MSM_REGIME_BATCH ? tune_batch_width(log_min) : 1;
@@ -122,7 +127,7 @@ int autotune(hzk_ctx* ctx, int regime, int group, int log_min, int log_max, doub
     const int cmax = MSM_MAX_C;
 
     for (int L = log_min; L <= log_max && !rc; ++L) {
-        const size_t n = (size_t)1 << L;
+        const size_t n = tune_points(L);
         const uint32_t B = regime == MSM_REGIME_BATCH ? tune_batch_width(L) : 1;
         const size_t step = n / 64 + 1;
         hzk_tune_entry& slot = ctx->tune[regime][group - 1][L];
@@ -132,7 +137,7 @@ int autotune(hzk_ctx* ctx, int regime, int group, int log_min, int log_max, doub
             return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_class).count() > budget_ms;
         };
         MsmPlan base = msm_plan_ctx(ctx, group - 1, n, 0, regime);
-        hzk_tune_entry best{base.c, base.K, base.g};
+        hzk_tune_entry best{base.c, base.K, base.g, true};
         slot = best;
         double tbest = time_msm(ctx, group, ds, db, n, B, step, dd, reps, &rc);
         auto try_entry = [&](hzk_tune_entry e) {
@@ -147,21 +152,21 @@ int autotune(hzk_ctx* ctx, int regime, int group, int log_min, int log_max, doub
         for (int c = base.c - 3; c <= base.c + 2; ++c) {
             if (c < MSM_MIN_C || c > cmax || c == base.c) continue;
             MsmPlan q = msm_plan(n, c, 0);
-            if (regime == MSM_REGIME_BATCH) try_entry({c, base.K, std::min<uint32_t>(base.g, 1u << (c - 1))});
-            else try_entry({c, q.K, q.g});
+            if (regime == MSM_REGIME_BATCH) try_entry({c, base.K, std::min<uint32_t>(base.g, 1u << (c - 1)), true});
+            else try_entry({c, q.K, q.g, true});
         }
         // 2. chunk length
         const hzk_tune_entry afterc = best;
         for (uint32_t K : {afterc.K / 4, afterc.K / 2, afterc.K * 2, afterc.K * 4}) {
             if (K < 4 || K % 4 || K > 4096) continue;
-            try_entry({afterc.c, K, afterc.g});
+            try_entry({afterc.c, K, afterc.g, true});
         }
         // 3. bucket-reduction run length
         const hzk_tune_entry afterk = best;
         for (uint32_t g = 1; g <= 64; g <<= 1) {
             if (g == afterk.g || g > (1u << (afterk.c - 1))) continue;
             if (regime == MSM_REGIME_SINGLE && g > 32) continue;
-            try_entry({afterk.c, afterk.K, g});
+            try_entry({afterk.c, afterk.K, g, true});
         }
         slot = best;
     }
@@ -190,6 +195,9 @@ int hzk_msm_batch_tune_set(hzk_ctx* ctx, int group, int log_n, int c, uint32_t K
 }
 int hzk_msm_batch_tune_get(hzk_ctx* ctx, int group, int log_n, int* c, uint32_t* K, uint32_t* g) {
     return tune_get(ctx, MSM_REGIME_BATCH, group, log_n, c, K, g);
+}
+int hzk_msm_tune_load(hzk_ctx* ctx, int batch, int group, int log_n, int c, uint32_t K, uint32_t g) {
+    return tune_set(ctx, batch ? MSM_REGIME_BATCH : MSM_REGIME_SINGLE, group, log_n, c, K, g, true);
 }
 int hzk_msm_batch_autotune(hzk_ctx* ctx, int group, int log_min, int log_max, double budget_ms) {
     return autotune(ctx, MSM_REGIME_BATCH, group, log_min, log_max, budget_ms);

@@ -41,9 +41,9 @@ def load(ctx, path=DEFAULT):
     n = 0
     for group, key in ((1, "g1"), (2, "g2")):
         for lg, (c, K, g) in table.get(key, {}).items():
-            ctx.msm_tune_set(group, int(lg), int(c), int(K), int(g))
+            ctx.msm_tune_load(group, int(lg), int(c), int(K), int(g))
             n += 1
         for lg, (c, K, g) in table.get(key + "_batch", {}).items():
-            ctx.msm_batch_tune_set(group, int(lg), int(c), int(K), int(g))
+            ctx.msm_tune_load(group, int(lg), int(c), int(K), int(g), batch=True)
             n += 1
     return n
