@@ -677,12 +677,13 @@ struct NttPlanPass { int s0, R, gl, hb; };
 // bytes or more, 1 where that saves a pass); the passes before it keep as
 // many columns. Otherwise the lowest min(k, TB) stages (contiguous rows) form
 // the last pass, the rest split evenly into passes of <= TB - 2 stages. A DIT
-// run executes the same passes in reverse order. k >= 3.
-static void plan_passes(int k, int TB, bool rev, std::vector<NttPlanPass>& out) {
-    out.clear();
+// run executes the same passes in reverse order. 3 <= k <= NTT_MAX_LOG, TB >= 9
+// or k <= TB; returns the number of passes.
+static constexpr int NTT_MAX_PASSES = 4;
+static int plan_passes(int k, int TB, bool rev, NttPlanPass* out) {
     if (k <= TB) {
-        out.push_back({0, k, 0, 0});
-        return;
+        out[0] = {0, k, 0, 0};
+        return 1;
     }
     const int last = rev ? 0 : TB, rest = k - last;
     int np = (rest + TB - 3) / (TB - 2);
@@ -691,14 +692,16 @@ static void plan_passes(int k, int TB, bool rev, std::vector<NttPlanPass>& out) 
     for (int p = 0; p < np; ++p) {
         const int R = rest / np + (p < rest % np ? 1 : 0);
         if (rev && p + 1 == np) {
-            out.push_back({s0, R, 0, std::min(TB - R, s0)});
-            return;
+            out[p] = {s0, R, 0, std::min(TB - R, s0)};
+            return np;
         }
-        out.push_back({s0, R, std::min(TB - R, k - s0 - R), 0});
+        out[p] = {s0, R, std::min(TB - R, k - s0 - R), 0};
         s0 += R;
     }
-    out.push_back({s0, last, 0, 0});
+    out[np] = {s0, last, 0, 0};
+    return np + 1;
 }
+static_assert((NTT_MAX_LOG - 9 + 6) / 7 + 1 <= NTT_MAX_PASSES && (NTT_MAX_LOG + 7) / 8 <= NTT_MAX_PASSES, "passes over tiles of 2^9");
 
 // elements per thread (2^LE) of a launch over `elems` elements: 4 while
 // that still gives every SIMD two waves, else 2 (more threads and more
@@ -721,13 +724,12 @@ static int tile_bits_for(hzk_ctx* ctx, uint64_t elems, int le) {
 // descriptor of *permute (k > 0) is left to k_ntt_permute.
 static void build_passes(fr_t* x, int k, int TB, bool dit, bool rev, const fr_t* tw, bool raw, const fr_t* pre, const fr_t* post,
                          const fr_t* scale, fr_t* ws, std::vector<NttPassDesc>& out, NttPassDesc* permute) {
-    std::vector<NttPlanPass> plan;
-    plan_passes(k, TB, rev && (ws || k <= TB), plan);
-    if (dit) std::reverse(plan.begin(), plan.end());
-    const size_t m = plan.size();
+    NttPlanPass plan[NTT_MAX_PASSES];
+    const int m = plan_passes(k, TB, rev && (ws || k <= TB), plan);
+    if (dit) std::reverse(plan, plan + m);
     const bool swap = rev && m > 1 && ws, later = rev && m > 1 && !ws;
     permute->k = 0;
-    for (size_t p = 0; p < m; ++p) {
+    for (int p = 0; p < m; ++p) {
         const bool first = p == 0, last = p + 1 == m;
         NttPassDesc d{};
         d.src = swap && !first ? ws : x;
@@ -867,8 +869,10 @@ int ntt_batch(hzk_ctx* ctx, const NttJob* jobs, size_t count, int capture) {
         if (jobs[i].kind <= 3 && k > TB) ws_elems += jobs[i].deg;
     }
     fr_t* const ws = ws_elems ? ntt_workspace(ctx, ws_elems) : nullptr;
-    // the passes of each transform; tiny ones and (without a workspace) permutations are launched singly
-    std::vector<std::vector<NttPassDesc>> passes(count);
+    // the passes of each transform, one after the other; tiny ones and (without a workspace) permutations are launched singly
+    std::vector<NttPassDesc> passes;
+    std::vector<size_t> pass_begin(count + 1, 0);
+    passes.reserve(2 * count);
     std::vector<NttPassDesc> tiny, permutes;
     size_t rounds = 0;
     uint64_t ws_at = 0;
@@ -879,6 +883,7 @@ int ntt_batch(hzk_ctx* ctx, const NttJob* jobs, size_t count, int capture) {
         const fr_t* post = kind == 3 ? t.coset[1] : kind == 6 ? t.coset_rev[1] : nullptr;
         const fr_t* scale = kind == 1 ? t.ninv : nullptr;
         fr_t* x = (fr_t*)jobs[i].x;
+        pass_begin[i + 1] = passes.size();
         if (ks[i] < 3) {
             NttPassDesc d{};
             d.src = d.dst = x, d.tw = t.tw[inv], d.pre = pre, d.post = post, d.scale = scale, d.k = ks[i];
@@ -891,23 +896,24 @@ int ntt_batch(hzk_ctx* ctx, const NttJob* jobs, size_t count, int capture) {
             w = ws + ws_at;
             ws_at += jobs[i].deg;
         }
-        build_passes(x, ks[i], TB, kind == 5, kind <= 3, t.tw[inv], false, pre, post, scale, w, passes[i], &permute);
+        build_passes(x, ks[i], TB, kind == 5, kind <= 3, t.tw[inv], false, pre, post, scale, w, passes, &permute);
         if (permute.k) permutes.push_back(permute);
-        rounds = std::max(rounds, passes[i].size());
+        pass_begin[i + 1] = passes.size();
+        rounds = std::max(rounds, pass_begin[i + 1] - pass_begin[i]);
     }
     // pass descriptors, round by round
     std::vector<NttPassDesc> pds;
+    pds.reserve(passes.size());
     std::vector<size_t> round_begin(rounds + 1, 0);
     std::vector<uint64_t> round_tiles(rounds, 0);
     for (size_t r = 0; r < rounds; ++r) {
         round_begin[r] = pds.size();
         uint64_t tiles = 0;
         for (size_t i = 0; i < count; ++i) {
-            if (r >= passes[i].size()) continue;
-            NttPassDesc d = passes[i][r];
-            d.tile_begin = tiles;
-            pds.push_back(d);
-            tiles += pass_tiles(d);
+            if (pass_begin[i] + r >= pass_begin[i + 1]) continue;
+            pds.push_back(passes[pass_begin[i] + r]);
+            pds.back().tile_begin = tiles;
+            tiles += pass_tiles(pds.back());
         }
         round_tiles[r] = tiles;
     }
