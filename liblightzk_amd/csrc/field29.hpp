@@ -148,8 +148,8 @@ struct g1acc29 {
     // a finite point's ZZ = Z^2 never is): a plain store, so a lane that
     // finishes a bucket in the middle of its chunk holds the others up for a
     // few instructions instead of four conversions. The later stages (bucket
-    // fix-up and reduction) read and write this form too; only the window
-    // sums leave it (to_xyzz).
+    // fix-up and reduction) read and write this form too, a coordinate per lane
+    // (LanePoint::load_raw); only the window sums leave it.
     static constexpr int RAW_WORDS = 36;
     HZK_DEV void to_words(uint32_t* w) const {
 #pragma unroll
@@ -173,15 +173,6 @@ struct g1acc29 {
         to_words(w);
 #pragma unroll
         for (int q = 0; q < RAW_WORDS / 4; ++q) dst[q] = make_uint4(w[4 * q], w[4 * q + 1], w[4 * q + 2], w[4 * q + 3]);
-    }
-    static HZK_DEV g1acc29 load_raw(const uint4* src) {
-        uint32_t w[RAW_WORDS];
-#pragma unroll
-        for (int q = 0; q < RAW_WORDS / 4; ++q) {
-            const uint4 v = src[q];
-            w[4 * q] = v.x, w[4 * q + 1] = v.y, w[4 * q + 2] = v.z, w[4 * q + 3] = v.w;
-        }
-        return from_words(w);
     }
 
     // this += q for two states under the bounds (add-2008-s); when q equals
@@ -306,7 +297,7 @@ struct g2acc29 {
         }
         finish(P, R, X, Y, ZZ, ZZZ, d);
     }
-    // raw state: 72 words, infinity has ZZ = 0 (read back by load_raw)
+    // raw state: 72 words, infinity has ZZ = 0 (read back by LanePoint::load_raw)
     static constexpr int RAW_WORDS = 72;
     HZK_DEV void to_words(uint32_t* w) const {
         const fq29* c[8] = {&X.c0, &X.c1, &Y.c0, &Y.c1, &ZZ.c0, &ZZ.c1, &ZZZ.c0, &ZZZ.c1};
@@ -333,15 +324,6 @@ struct g2acc29 {
         to_words(w);
 #pragma unroll
         for (int q = 0; q < RAW_WORDS / 4; ++q) dst[q] = make_uint4(w[4 * q], w[4 * q + 1], w[4 * q + 2], w[4 * q + 3]);
-    }
-    static HZK_DEV g2acc29 load_raw(const uint4* src) {
-        uint32_t w[RAW_WORDS];
-#pragma unroll
-        for (int q = 0; q < RAW_WORDS / 4; ++q) {
-            const uint4 v = src[q];
-            w[4 * q] = v.x, w[4 * q + 1] = v.y, w[4 * q + 2] = v.z, w[4 * q + 3] = v.w;
-        }
-        return from_words(w);
     }
     // the R = 2^256 XYZZ point (canonical components; infinity = all zero)
     HZK_DEV xyzz_t<fq2_t> to_xyzz() const {
