@@ -1,14 +1,14 @@
-// Fr in nine 29-bit limbs (fr29), for the NTT's latency-bound two-element
-// passes (ntt.hip). Needs HZK_DEV and fr_t (eight 32-bit limbs, field.hpp)
-// declared first; plain C++ otherwise, so the host sanitizer build checks it
-// against the oracle's Fr product.
+// Fr in nine 29-bit limbs: fr29 (unsigned, one reduction per product) for the
+// NTT's smallest transforms and its separate permutation, and the reduction that
+// ends its passes on signed limbs (fr_reduce). Needs HZK_DEV and fr_t (eight
+// 32-bit limbs, field.hpp) declared first; plain C++ otherwise, so host builds
+// check it against the oracle's Fr product and against integers.
 #pragma once
 #include <cstdint>
 
 namespace hzk {
 
-// Fr in nine 29-bit limbs for the latency-bound two-element passes. The
-// boundary form's Montgomery product (field.hpp: eight 32-bit limbs, one
+// The boundary form's Montgomery product (field.hpp: eight 32-bit limbs, one
 // chain of 128 multiply-adds with carry folds) is a long dependency chain;
 // here the 17 product columns are independent sums (a 64-bit column cannot
 // overflow), and only the nine reduction digits form a chain of a few

@@ -82,8 +82,9 @@ template <class F> struct LaneOf;
 template <> struct LaneOf<fq_t> { using T = LaneFq; };
 template <> struct LaneOf<fq2_t> { using T = LaneFq2; };
 
-// the lane's coordinate of an accumulator (bounds as in g1acc29), normalized;
-// inf is the same in every lane of the group
+// the lane's coordinate of an accumulator (bounds as in g1acc29, Y in (-2, 2):
+// here it is the difference of two reduced products), normalized; inf is the
+// same in every lane of the group
 template <class F>
 struct LanePoint {
     using L = typename LaneOf<F>::T;

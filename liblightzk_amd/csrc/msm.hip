@@ -26,7 +26,7 @@
 //              piece scatters. A group that one digit value fills (the ones of
 //              a witness) is many pieces, so no workgroup has more to do than
 //              the others; a histogram over all buckets of a window is never
-//              needed, so windows may have 2^19 buckets.
+//              needed, so a window may have more buckets than LDS has counters.
 //  1'-4'. instances of at most MSM_SMALL_N points with few buckets: the recode,
 //              then one workgroup per window sorts it whole in LDS.
 //  5-8 (msm_impl.hpp) chunked accumulation with boundary fix-up, bucket

@@ -11,7 +11,7 @@ namespace hzk {
 
 constexpr int MSM_MIN_C = 4;
 constexpr int MSM_MAX_C = 16;         // a caller's window sizes and the autotuner's
-constexpr int MSM_PLAN_MAX_C = 20;    // built-in plans
+constexpr int MSM_PLAN_MAX_C = 17;    // tuned plans (msm_widen)
 
 struct MsmPlan {
     int c;          // window bits
@@ -21,13 +21,15 @@ struct MsmPlan {
     uint32_t g;     // buckets per bucket-reduction run
     bool fit = false;   // a tuned plan (built in, autotuned or loaded): msm_fit_chunks may move K, msm_widen c
 };
-// Tuned plans (size classes up to 2^24) from MSM_WIDE_N G1 points on take 17-bit windows, one more
-// than a caller may ask for: 15 of them instead of 16 save that part of the
+// Tuned plans from MSM_WIDE_N G1 points on take 17-bit windows, one more than a
+// caller may ask for: 15 of them instead of 16 save that part of the
 // accumulation and the sort, for twice the buckets: 2^23 points 10.89 -> 10.45
 // ms, 2^24 20.83 -> 20.14, 7 million 9.11 -> 8.89; 2^22 and less gain under 1 %.
+// From 2^25 points on, above the classes of the shipped table, plans are the
+// heuristic's (16 bits) unless a tuned one is loaded.
 constexpr size_t MSM_WIDE_N = (size_t)1 << 22;
 inline void msm_widen(int g2, size_t n, MsmPlan& p) {
-    if (!g2 && p.c == 16 && n >= MSM_WIDE_N) p.c = 17, p.W = 15, p.NB = 1u << 16;
+    if (!g2 && p.c == 16 && n >= MSM_WIDE_N) p.c = MSM_PLAN_MAX_C, p.W = 15, p.NB = 1u << 16;
 }
 // Plan for n points: autotuned entry for the size class if one is loaded,
 // else the built-in heuristic; force_c / force_g override (0 = automatic).

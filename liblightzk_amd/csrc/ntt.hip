@@ -124,8 +124,8 @@ HZK_DEV void fr_mul2(limbs29& r0, const limbs29& a0, const limbs29& b0, limbs29&
 
 // LDS slot of tile element e: two 16-byte planes and a 4-byte one (limbs 0-3,
 // 4-7, 8), so lanes reading consecutive elements touch consecutive words; the
-// low 3 bits are XOR-ed with the next 3 so that threads holding 8 consecutive
-// elements (the lowest radix-8 group) spread over the banks
+// low 3 bits are XOR-ed with the next 3 so that lanes that hold 4 (or 2)
+// consecutive elements each, in the lowest stages, spread over the banks
 HZK_DEV uint32_t lds_slot(uint32_t e) { return e ^ ((e >> 3) & 7); }
 template <int TB>
 constexpr int ntt_lds_vecs() { return (2 << TB) + (1 << (TB - 2)); }   // uint4 of a tile's LDS
@@ -191,7 +191,7 @@ struct NttTile {
 // first pairs (0, 2) and (1, 3) with twiddles w0, w1, the second (0, 1) and
 // (2, 3), both with w2. A product's operand may hold a sum or difference of
 // two normalized values; elements leave normalized. One product at a time:
-// four waves share the SIMD, and the registers saved are what lets them.
+// three waves share the SIMD, and the registers saved are what lets them.
 HZK_DEV void ntt_dif2(limbs29* v, const fr_t& t0, const fr_t& t1, const fr_t& t2, int flags) {
     limbs29 d = v[0] - v[2], e = v[1] - v[3];
     v[0] = v[0] + v[2];
